@@ -38,13 +38,11 @@
 //                   few long rows (fewer than about two per CU): each row cut
 //                   into slices over the CUs, one partial maximum per slice
 //                   in the workspace, then the cast of each slice
-//   k_quant_cols_1pass
-//                   per-column (axis 1) quant in one launch for rows of 8192,
-//                   16384 or 32768 elements and x of 2^22 elements up to
-//                   480 MiB: k_quant_tensor_1pass's step layout with running
-//                   column maxima per thread, then two grid-wide exchanges
-//                   (partial column maxima; each workgroup's slice of
-//                   multipliers) and the cast from registers / LDS
+//   k_quant_cols_strip
+//                   per-column (axis 1) quant in one launch for rows of a
+//                   multiple of 8 elements and x of up to 480 MiB: strips of
+//                   columns x row blocks held in registers / LDS, one
+//                   grid-wide exchange of the partial column maxima
 //   k_colmax / k_col_finalize / k_cast_cols
 //                   per-column (axis 1) quant otherwise: partial column
 //                   maxima per row block, one finalize pass, then the cast
@@ -532,146 +530,102 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_tensor_1pass(
 }
 
 // ---------------------------------------------------------------------------
-// Per column (axis 1) in one launch, for rows of 8192, 16384 or 32768
-// elements (c8 = cols / 8 = 1024 CPT chunks, CPT = 1, 2 or 4) and x of up to
-// CBQ_COLS_1PASS_MAX_BYTES (the host checks both). The step
-// layout of k_quant_tensor_1pass: a resident grid of G workgroups (a power
-// of two) reads x once in grid-wide steps of G x 4096 chunks, holding the
-// last HS steps of each thread in registers and parking the first LS streamed
-// steps in LDS (128 MiB of 2-byte x in all on 256 CUs); since a step starts
-// at a multiple of c8 chunks, chunk u of thread t is always of chunk-column
-// t + 1024 (u % CPT), so each thread keeps the running |x| maxima of its CPT
-// chunk-columns (8 columns each). Then two grid-wide exchanges through the
-// workspace:
-//  1. every workgroup stores its [cols] partial maxima (part[b], in planes
-//     of 64-bit words: a wave's stores cover 512 contiguous bytes; with
-//     8-byte stores 32 bytes apart the exchange ran at under 1 TB/s; 16-bit
-//     values of the input dtype for 2-byte input, see st8_max) and
-//     publishes its slot with tag T1; once every slot carries T1 (or T2),
-//     workgroup b reduces the partials of its slice of c8 / G chunk-columns
-//     (<= 16) over all G workgroups, stores the slice's multipliers inv[c] =
-//     fp32(127 / max(amax_c, eps)) and publishes T2;
-//  2. once every slot carries T2, every thread loads the multipliers of its
-//     chunk-columns and casts its held steps from registers, the parked ones
-//     from LDS, and re-reads the rest; workgroup b writes its slice's scales.
-// HBM traffic 2N (+ the re-read beyond 128 MiB) + N + the partial maxima
-// (2 G cols bytes for 2-byte input, 4 G cols for fp32, each written and read
-// once), against 2N + 2N + N for k_colmax + k_cast_cols.
+// Per column (axis 1) in one launch: k_quant_cols_strip, for x whose rows are
+// a multiple of 8 elements (16-byte aligned x).
 //
-// Tags and timeouts follow the per-tensor exchange (the same control block:
-// gen, status, suspect, slots). T1 = gen + 1 and T2 = T1 + 1 (skipping 0);
-// only a workgroup whose second wait completed advances gen (workgroup 0, or
-// any of them once suspect holds T1 or T2). A workgroup that gives up on the
-// first wait publishes NaN multipliers for its slice (so those columns get a
-// NaN scale and 0 codes everywhere); one that gives up on the second writes 0
-// codes, and then every workgroup that completes the second wait finds
-// suspect == T2 and writes NaN scales. A scale that is not NaN therefore
-// comes with every code of its column exact.
+// The matrix is cut into strips of SW = 2^sl chunks (8 columns each; 64
+// chunks = 1 KiB of 2-byte elements per row) and each strip into row blocks;
+// a resident grid of at most one workgroup per CU takes one (strip, row block)
+// each and reads it once, 64 bytes per thread in flight: thread t always
+// chunk-column t % SW of rows t / SW, + 1024 / SW, ..., so it keeps the eight
+// running |x| maxima of its chunk-column. The last six 64-byte steps (fp32:
+// five) stay in registers, the first two streamed ones in LDS (128 MiB of x
+// in all on 256 CUs), what does not fit is read again for the cast.
+//
+// Exchange: the workgroup's column maxima (LDS atomics, then 16-bit values
+// of the input dtype for 2-byte input) go to part[strip][row block], the
+// workgroup publishes its slot, waits for the others and reduces its own
+// strip's row blocks (SW x row blocks values: 32 KiB for [11008, 4096]). One
+// wait and one launch replace column maxima + finalize + cast, which read x
+// twice (bf16 [11008, 4096], kernels: 17.6 + 5.8 + 22.8 us). A matrix whose
+// strips have one row block each needs no exchange.
+//
+// Bound: memory (x once and the codes, plus the partial maxima) up to 128 MiB of x.
+//
+// Tags follow the per-tensor exchange (the same control block: gen, status,
+// suspect, slots; one tag per call). A workgroup whose wait gives up does not
+// need the others: it takes the maxima of its strip from x itself and goes
+// on, so every result is exact however the workgroups are scheduled (two
+// such grids on two streams may each hold some of the CUs); it still sets
+// status, and suspect so that a workgroup that completes advances gen (the
+// last workgroup to publish always completes). Waits are therefore short:
+// kColsSpinLimit polls at most.
 // ---------------------------------------------------------------------------
-constexpr int kColsMaxSlice = 16;   // chunk-columns per workgroup in the slice reduction
-constexpr int64_t kColsMinElems = int64_t(1) << 22;
-// Largest x (bytes) the one-launch column path takes; larger ones take
-// k_colmax + k_cast_cols. Measured on MI355X (bf16, cols 8192, op time after
-// a cache sweep, one-launch against two-pass, same process): 64 MiB 32.6 /
-// 37.8 us, 128 MiB 48.4 / 62.4, 256 MiB 101.6 / 112.2, 384 MiB 154.2 /
-// 159.3, 448 MiB 182.2 / 184.0, 576 MiB 235.7 / 232.9 us: past what
-// registers and LDS hold (128 MiB) the re-read of the rest and the exchange
-// cost about what the single read saves. A compile-time tuning knob.
+constexpr int kColsMaxSL = 6;                     // strips of at most 64 chunks
+// Chunks in flight per thread (64 bytes), steps of that many held in
+// registers (six: 96 VGPRs; fp32 five, whose maxima take twice the registers)
+// and parked in LDS.
+template <int DT> constexpr int strip_u() { return DT == kF32 ? 2 : 4; }
+template <int DT> constexpr int strip_hold() { return DT == kF32 ? 5 : 6; }
+constexpr int kStripPark = 2;
+constexpr uint32_t kColsSpinLimit = 4096;         // polls, a few milliseconds
+// Largest x (bytes) of the one-launch column path; larger ones take
+// k_colmax + k_cast_cols. A compile-time tuning knob.
 #ifndef CBQ_COLS_1PASS_MAX_BYTES
 #define CBQ_COLS_1PASS_MAX_BYTES (int64_t(480) << 20)
 #endif
 
-// Steps held in registers: those of k_quant_tensor_1pass, less what the CPT
-// chunk-columns' 8 maxima (then multipliers) per thread take.
-template <int DT, int CPT>
-constexpr int cols_hold_steps() {
-  return DT == kF32 ? (CPT == 1 ? 3 : CPT == 2 ? 2 : 1) : (CPT == 1 ? 6 : CPT == 2 ? 5 : 3);
-}
-
 __device__ __forceinline__ uint32_t next_tag(uint32_t g) { return g + 1 == 0 ? 1u : g + 1; }
 
-// Agent-scope 64-bit accesses (coherent across the XCDs' L2s, like the
-// slots) to the exchange arrays, which hold 8 floats per chunk-column as 4
-// planes of pairs: element (i, c) = floats 2i, 2i + 1 of chunk-column c, so
-// that the 64 lanes of a wave (consecutive c) access 512 contiguous bytes.
-__device__ __forceinline__ void ld8_pairs(const unsigned long long* p, int64_t plane,
-                                          int64_t c, float (&v)[8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned long long d =
-        __hip_atomic_load(p + i * plane + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    v[2 * i] = __uint_as_float(static_cast<uint32_t>(d));
-    v[2 * i + 1] = __uint_as_float(static_cast<uint32_t>(d >> 32));
-  }
-}
-
-__device__ __forceinline__ void st8_pairs(unsigned long long* p, int64_t plane, int64_t c,
-                                          const float (&v)[8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    __hip_atomic_store(p + i * plane + c,
-                       static_cast<unsigned long long>(__float_as_uint(v[2 * i])) |
-                           (static_cast<unsigned long long>(__float_as_uint(v[2 * i + 1])) << 32),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // The column maxima of one chunk-column (8 columns) as they cross the
-// exchange: for 2-byte input as the input dtype's 16-bit values, 4 per
-// 64-bit word in 2 planes (each maximum is the absolute value of an input
-// element, so it is exact in that dtype; half the bytes of fp32), for fp32
-// input as fp32 pairs in 4 planes.
+// exchange: a chunk of the input dtype (each maximum is the absolute value of
+// an input element, so it is exact there), in NP planes of 64-bit words (2 for
+// 2-byte input, 4 for fp32), so that the 64 lanes of a wave (consecutive c)
+// access 512 contiguous bytes; agent-scope accesses (coherent across the XCDs'
+// L2s, like the slots).
 template <int DT> constexpr int max_planes() { return DT == kF32 ? 4 : 2; }
 
 template <int DT>
-__device__ __forceinline__ uint32_t max_to16(float f) {
-  if constexpr (DT == kBF16) return __float_as_uint(f) >> 16;
+__device__ __forceinline__ uint32_t max_bits(float f) {
+  if constexpr (DT == kF32) return __float_as_uint(f);
+  else if constexpr (DT == kBF16) return __float_as_uint(f) >> 16;
   else return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
-}
-
-template <int DT>
-__device__ __forceinline__ float max_from16(uint32_t h) {
-  if constexpr (DT == kBF16) return __uint_as_float(h << 16);
-  else return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h)));
 }
 
 template <int DT>
 __device__ __forceinline__ void st8_max(unsigned long long* p, int64_t plane, int64_t c,
                                         const float (&v)[8]) {
-  if constexpr (DT == kF32) {
-    st8_pairs(p, plane, c, v);
-  } else {
+  constexpr int PW = DT == kF32 ? 2 : 4;   // values per word
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      unsigned long long w = 0;
+  for (int i = 0; i < max_planes<DT>(); ++i) {
+    unsigned long long w = 0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        w |= static_cast<unsigned long long>(max_to16<DT>(v[4 * i + j])) << (16 * j);
-      __hip_atomic_store(p + i * plane + c, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    for (int j = 0; j < PW; ++j)
+      w |= static_cast<unsigned long long>(max_bits<DT>(v[PW * i + j])) << (64 / PW * j);
+    __hip_atomic_store(p + i * plane + c, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
 template <int DT>
-__device__ __forceinline__ void ld8_max(const unsigned long long* p, int64_t plane, int64_t c,
-                                        float (&v)[8]) {
-  if constexpr (DT == kF32) {
-    ld8_pairs(p, plane, c, v);
-  } else {
+__device__ __forceinline__ Raw8<DT> ld8_max(const unsigned long long* p, int64_t plane, int64_t c) {
+  uint32_t w[2 * max_planes<DT>()];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const unsigned long long w =
-          __hip_atomic_load(p + i * plane + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        v[4 * i + j] = max_from16<DT>(static_cast<uint32_t>(w >> (16 * j)) & 0xffffu);
-    }
+  for (int i = 0; i < max_planes<DT>(); ++i) {
+    const unsigned long long d =
+        __hip_atomic_load(p + i * plane + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    w[2 * i] = static_cast<uint32_t>(d);
+    w[2 * i + 1] = static_cast<uint32_t>(d >> 32);
   }
+  Raw8<DT> r;
+  r.a = make_uint4(w[0], w[1], w[2], w[3]);
+  if constexpr (DT == kF32) r.b = make_uint4(w[4], w[5], w[6], w[7]);
+  return r;
 }
 
-// Waits until every slot [0, G) carries tag or alt; after spin_limit polls
+// Waits until every slot [0, G) carries tag; after spin_limit polls
 // records suspect = tag and status = 1 (both performed before it) and polls
 // once more. Returns whether the wait completed (every thread gets it).
-__device__ int slot_wait(char* ctl, uint32_t tag, uint32_t alt, uint32_t spin_limit) {
+__device__ int slot_wait(char* ctl, uint32_t tag, uint32_t spin_limit) {
   auto* slots = reinterpret_cast<unsigned long long*>(ctl + kCtlSlots);
   const int G = static_cast<int>(gridDim.x);
   auto poll = [&]() {
@@ -679,7 +633,7 @@ __device__ int slot_wait(char* ctl, uint32_t tag, uint32_t alt, uint32_t spin_li
     for (int i = threadIdx.x; i < G; i += blockDim.x) {
       const uint32_t t = static_cast<uint32_t>(
           __hip_atomic_load(slots + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32);
-      ok &= (t == tag) | (t == alt);
+      ok &= t == tag;
     }
     return __syncthreads_and(ok);
   };
@@ -724,13 +678,57 @@ __device__ __forceinline__ void slot_publish(char* ctl, uint32_t tag, bool refre
   __syncthreads();
 }
 
-template <int DT, int CPT>
-__device__ __forceinline__ void colmax8(const Raw8<DT>& r, float (&m)[8]) {
-  float f[8];
-  cvt8<DT>(r, f);
+// Running |x| maxima of the 8 columns of a chunk-column, NaN ignored. fp32: 8
+// floats. 2-byte types: packed 16-bit integers, half the registers and
+// three operations per pair: |x|'s bits plus a bias that moves infinity to
+// 0x7fff order like the values, and a NaN's become negative and lose the signed
+// maximum against the start value, the bias (|x| = 0).
+template <int DT>
+struct ColMax {
+  static constexpr uint32_t kBias = DT == kBF16 ? 0x007f007fu : 0x03ff03ffu;
+  typedef short s16x2 __attribute__((ext_vector_type(2)));
+  s16x2 m[4] = {__builtin_bit_cast(s16x2, kBias), __builtin_bit_cast(s16x2, kBias),
+                __builtin_bit_cast(s16x2, kBias), __builtin_bit_cast(s16x2, kBias)};
+  __device__ __forceinline__ void add(const Raw8<DT>& r) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const uint32_t w[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
 #pragma unroll
-  for (int e = 0; e < 8; ++e) m[e] = fmaxf(m[e], __builtin_fabsf(f[e]));
-}
+    for (int k = 0; k < 4; ++k) {
+      const u16x2 v = __builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu) + __builtin_bit_cast(u16x2, kBias);
+      m[k] = __builtin_elementwise_max(m[k], __builtin_bit_cast(s16x2, v));
+    }
+  }
+  // over the lanes l, l ^ o, l ^ 2o, ... of the wave
+  __device__ __forceinline__ void across(int o) {
+    for (; o < kWave; o <<= 1)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        m[k] = __builtin_elementwise_max(
+            m[k], __builtin_bit_cast(s16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), o)));
+  }
+  __device__ __forceinline__ float get(int e) const {
+    const uint32_t w = __builtin_bit_cast(uint32_t, m[e >> 1]) - kBias;   // no borrow: m >= bias
+    const uint32_t h = (e & 1) ? w >> 16 : w & 0xffffu;
+    if constexpr (DT == kBF16) return __uint_as_float(h << 16);
+    else return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h)));
+  }
+};
+template <>
+struct ColMax<kF32> {
+  float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  __device__ __forceinline__ void add(const Raw8<kF32>& r) {
+    float f[8];
+    cvt8<kF32>(r, f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m[e] = fmaxf(m[e], __builtin_fabsf(f[e]));
+  }
+  __device__ __forceinline__ void across(int o) {
+    for (; o < kWave; o <<= 1)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m[e] = fmaxf(m[e], __shfl_xor(m[e], o));
+  }
+  __device__ __forceinline__ float get(int e) const { return m[e]; }
+};
 
 template <int DT>
 __device__ __forceinline__ uint2 cast8_cols(const Raw8<DT>& r, const float (&inv)[8]) {
@@ -741,184 +739,169 @@ __device__ __forceinline__ uint2 cast8_cols(const Raw8<DT>& r, const float (&inv
   return pack8_int8(f, 1.0f);   // x 1: exact
 }
 
-template <int DT, int CPT>
-__global__ __launch_bounds__(kFusedBlock) void k_quant_cols_1pass(
-    const void* __restrict__ x, int64_t n8, float eps, int8_t* __restrict__ q,
-    float* __restrict__ scale_out, char* __restrict__ ctl, float* __restrict__ part,
-    float* __restrict__ invs, uint32_t spin_limit) {
-  constexpr int U = kFusedU;
-  constexpr int HS = cols_hold_steps<DT, CPT>();
-  constexpr int LS = fused_lds_steps<DT>();
+// Workgroup b: strip b % strips, row block b / strips (rows RB per block), so
+// that the workgroups running together read whole rows.
+template <int DT>
+__global__ __launch_bounds__(kFusedBlock) void k_quant_cols_strip(
+    const void* __restrict__ x, int64_t rows, int c8, int sl, int strips, int nrb, int64_t RB,
+    float eps, int8_t* __restrict__ q, float* __restrict__ scale_out, char* __restrict__ ctl,
+    unsigned long long* __restrict__ part, uint32_t spin_limit) {
+  constexpr int U = strip_u<DT>();
+  constexpr int HS = strip_hold<DT>();
+  constexpr int LS = kStripPark;
   constexpr int EB = 8 * elem_bytes<DT>();            // bytes of x per chunk
   constexpr int QW = EB / 16;                         // 16-byte words per chunk
-  constexpr int C8 = 1024 * CPT;                      // chunk-columns
-  static_assert(U % CPT == 0, "chunk u of a thread is of chunk-column t + 1024 (u % CPT)");
+  constexpr int NP = max_planes<DT>();
   __shared__ u32x4 park[LS * U * QW * kFusedBlock];
-  __shared__ float red[(kFusedBlock / kWave) * kColsMaxSlice * 8];
-  __shared__ uint32_t s_t1;
-  __shared__ int s_nan;
+  __shared__ unsigned int smax[2][8 << kColsMaxSL];   // [8 columns of a chunk][SW], as float bits
+  __shared__ uint32_t s_tag;
 
-  const int G = static_cast<int>(gridDim.x), b = static_cast<int>(blockIdx.x);
-  const int t = static_cast<int>(threadIdx.x), lane = t % kWave, wave = t / kWave;
-  auto* gen_w = reinterpret_cast<unsigned long long*>(ctl + kCtlGen);
-  auto* suspect = reinterpret_cast<unsigned int*>(ctl + kCtlSuspect);
-  if (t == 0)
-    s_t1 = next_tag(static_cast<uint32_t>(
-        __hip_atomic_load(gen_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+  const int b = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
+  const int SW = 1 << sl, rps = kFusedBlock >> sl;    // chunks per strip row, rows per chunk slot
+  const int strip = b % strips, rb = b / strips;
+  const int cc = t & (SW - 1), tr = t >> sl;
+  const bool col_ok = strip * SW + cc < c8;
+  const int64_t r0 = rb * RB, r1 = min(r0 + RB, rows);
+  const int64_t pitch = static_cast<int64_t>(c8) * EB;
+  if (t == 0 && nrb > 1)
+    s_tag = next_tag(static_cast<uint32_t>(
+        __hip_atomic_load(reinterpret_cast<unsigned long long*>(ctl + kCtlGen), __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_AGENT)));
+  for (int i = t; i < 2 * (8 << kColsMaxSL); i += kFusedBlock) (&smax[0][0])[i] = 0u;
 
-  const int64_t SB = static_cast<int64_t>(kFusedBlock) * U;   // chunks per workgroup and step
-  const int64_t GS = static_cast<int64_t>(G) * SB;            // chunks per grid step
-  const int64_t I = (n8 + GS - 1) / GS;
-  const int64_t held0 = I > HS ? I - HS : 0;
-  const char* xw = static_cast<const char*>(x) + static_cast<int64_t>(b) * SB * EB;
-  int8_t* qw = q + static_cast<int64_t>(b) * SB * 8;
-  const uint32_t xo = t * EB, qo = t * 8;
+  // Chunk slot j (rows r0 + j rps + tr) through a buffer resource based at
+  // its first row and ending with the strip in the block's last row: rows past
+  // the block read zeros and their stores are dropped; columns past the matrix
+  // get an offset beyond any end (the host keeps a block below 2^31 bytes).
+  const int64_t sb = min(static_cast<int64_t>(SW), static_cast<int64_t>(c8) - static_cast<int64_t>(strip) * SW) * EB;
+  const int64_t xe = (r1 - r0 - 1) * pitch + sb;
+  const int64_t xs = static_cast<int64_t>(rps) * pitch;       // bytes of x per chunk slot
+  const char* const xb = static_cast<const char*>(x) + r0 * pitch + static_cast<int64_t>(strip) * SW * EB;
+  int8_t* const qb = q + (r0 * c8 + static_cast<int64_t>(strip) * SW) * 8;
+  const uint32_t qv = (col_ok ? 0u : 0x40000000u) + (static_cast<uint32_t>(tr) * c8 + cc) * 8;
+  const uint32_t xv = col_ok ? qv * elem_bytes<DT>() : 0x80000000u;
+  auto load = [&](int j) {
+    const int64_t left = xe - j * xs;
+    return ld8_buf<DT>(__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(xb + j * xs), 0,
+                                                         static_cast<int>(left > 0 ? left : 0),
+                                                         kBufDword3), xv);
+  };
+  const int I = static_cast<int>((r1 - r0 + static_cast<int64_t>(rps) * U - 1) / (static_cast<int64_t>(rps) * U));
+  const int held0 = I > HS ? I - HS : 0;
 
-  // Pass 1: column maxima; streamed steps (the first LS parked), then the
-  // held steps into r[].
-  float m[CPT][8];
-#pragma unroll
-  for (int s = 0; s < CPT; ++s)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) m[s][e] = 0.0f;
-  for (int64_t i = 0; i < held0; ++i) {
+  // Pass 1: column maxima.
+  ColMax<DT> m;
+  for (int i = 0; i < held0; ++i) {
     Raw8<DT> v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = ld8_at<DT>(xw + (i * GS + u * kFusedBlock) * EB, xo);
+    for (int u = 0; u < U; ++u) v[u] = load(i * U + u);
 #pragma unroll
-    for (int u = 0; u < U; ++u) colmax8<DT, CPT>(v[u], m[u % CPT]);
+    for (int u = 0; u < U; ++u) m.add(v[u]);
     if (i < LS) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        u32x4* pk = park + (static_cast<int>(i) * U + u) * QW * kFusedBlock + t;
+        u32x4* pk = park + (i * U + u) * QW * kFusedBlock + t;
         pk[0] = u32x4{v[u].a.x, v[u].a.y, v[u].a.z, v[u].a.w};
         if constexpr (DT == kF32) pk[kFusedBlock] = u32x4{v[u].b.x, v[u].b.y, v[u].b.z, v[u].b.w};
       }
     }
   }
-  const int64_t cb = static_cast<int64_t>(b) * SB;
   Raw8<DT> r[HS * U];
 #pragma unroll
   for (int k = 0; k < HS; ++k) {
-    const int64_t c0 = (held0 + k) * GS + cb;
-    const int64_t left = n8 - c0;
-    __builtin_amdgcn_sched_barrier(0);
-    if (left > 0) {
-      const auto rs = rsrc(static_cast<const char*>(x) + c0 * EB, (left < SB ? left : SB) * EB);
+    __builtin_amdgcn_sched_barrier(0);   // one step's loads in flight at a time
+    if (held0 + k < I) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) r[k * U + u] = ld8_buf<DT>(rs, u * kFusedBlock * EB + xo);
+      for (int u = 0; u < U; ++u) r[k * U + u] = load((held0 + k) * U + u);
 #pragma unroll
-      for (int u = 0; u < U; ++u) colmax8<DT, CPT>(r[k * U + u], m[u % CPT]);
+      for (int u = 0; u < U; ++u) m.add(r[k * U + u]);
     }
   }
 #pragma unroll
   for (int j = 0; j < HS * U; ++j) reload_barrier<DT>(r[j]);
-
-  // Exchange 1: this workgroup's partial maxima (part: [G][NP planes][C8]
-  // words), then tag T1.
-  constexpr int NP = max_planes<DT>();
-  auto* part64 = reinterpret_cast<unsigned long long*>(part);
-  auto* inv64 = reinterpret_cast<unsigned long long*>(invs);   // [4 planes][C8] pairs
+  m.across(SW);                          // one lane per chunk-column and wave
+  __syncthreads();                       // smax is cleared
+  if (t % kWave < SW) {
 #pragma unroll
-  for (int s = 0; s < CPT; ++s)
-    st8_max<DT>(part64 + static_cast<int64_t>(b) * NP * C8, C8, t + 1024 * s, m[s]);
-  __builtin_amdgcn_s_waitcnt(0);
+    for (int e = 0; e < 8; ++e) atomicMax(&smax[0][e * SW + cc], __float_as_uint(m.get(e)));
+  }
   __syncthreads();
-  const uint32_t T1 = s_t1, T2 = next_tag(T1);
-  slot_publish(ctl, T1, false);
-  const int ok1 = slot_wait(ctl, T1, T2, spin_limit);
 
-  // Slice reduction: chunk-columns [b SCC, b SCC + SCC) over the G partials.
-  // Thread t takes chunk-column cc = t % SCC of partials (t + 1024 j) / SCC,
-  // then the lanes of a wave with the same cc combine (xor shuffles), then
-  // the waves through LDS.
-  const int SCC = C8 / G;                             // power of two, <= kColsMaxSlice
-  const int cc = t & (SCC - 1);
-  float sm[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) sm[e] = 0.0f;
-  if (ok1) {
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      const int p = (t + 1024 * j) / SCC;             // < G: G * SCC = C8 = 1024 CPT
+  // Exchange with the strip's other row blocks; smax[1] becomes the strip's
+  // column maxima.
+  if (nrb > 1) {
+    unsigned long long* const sp = part + static_cast<int64_t>(strip) * nrb * NP * SW;
+    if (t < SW) {
       float v[8];
-      ld8_max<DT>(part64 + static_cast<int64_t>(p) * NP * C8, C8, b * SCC + cc, v);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sm[e] = fmaxf(sm[e], v[e]);
+      for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(smax[0][e * SW + t]);
+      st8_max<DT>(sp + static_cast<int64_t>(rb) * NP * SW, SW, t, v);
     }
-  }
-  for (int o = SCC; o < kWave; o <<= 1)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sm[e] = fmaxf(sm[e], __shfl_xor(sm[e], o));
-  if (lane < SCC) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) red[(wave * SCC + lane) * 8 + e] = sm[e];
-  }
-  __syncthreads();
-  float inv_mine = 0.0f;                              // thread t < 8 SCC: column 8 (b SCC) + t
-  if (t < 8 * SCC) {
-    float mx = 0.0f;
-    for (int w = 0; w < kFusedBlock / kWave; ++w) mx = fmaxf(mx, red[(w * SCC + (t >> 3)) * 8 + (t & 7)]);
-    inv_mine = ok1 ? inv_scale(mx, eps, kQmaxInt8) : __builtin_nanf("");
-    // column 8 (b SCC + t / 8) + t % 8: plane (t % 8) / 2, half t % 2 of the pair
-    __hip_atomic_store(reinterpret_cast<unsigned int*>(inv64 + ((t & 7) >> 1) * C8 + b * SCC + (t >> 3)) +
-                           (t & 1),
-                       __float_as_uint(inv_mine), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  slot_publish(ctl, T2, true);
-  const int ok2 = slot_wait(ctl, T2, T2, spin_limit);
-  if (t == 0) {
-    int nan = !ok2;
-    if (ok2) {
-      const uint32_t sp = __hip_atomic_load(suspect, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (b == 0 || sp == T1 || sp == T2)
-        __hip_atomic_store(gen_w, static_cast<unsigned long long>(T2), __ATOMIC_RELAXED,
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    const uint32_t tag = s_tag;
+    slot_publish(ctl, tag, true);
+    const int ok = slot_wait(ctl, tag, spin_limit);
+    if (t == 0 && ok) {
+      auto* gen_w = reinterpret_cast<unsigned long long*>(ctl + kCtlGen);
+      auto* suspect = reinterpret_cast<unsigned int*>(ctl + kCtlSuspect);
+      const uint32_t su = __hip_atomic_load(suspect, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (b == 0 || su == tag)
+        __hip_atomic_store(gen_w, static_cast<unsigned long long>(tag), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
-      nan = sp == T2;
-      if (b == 0 && sp != 0 && sp != T1 && sp != T2) {   // an earlier call's record
-        uint32_t expect = sp;
+      if (b == 0 && su != 0 && su != tag) {   // an earlier call's record
+        uint32_t expect = su;
         __hip_atomic_compare_exchange_strong(suspect, &expect, 0u, __ATOMIC_RELAXED,
                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-    s_nan = nan;
+    ColMax<DT> all;
+    if (ok) {
+      for (int p = tr; p < nrb; p += rps)
+        all.add(ld8_max<DT>(sp + static_cast<int64_t>(p) * NP * SW, SW, cc));
+    } else if (col_ok) {
+      // gave up waiting: the strip's maxima from x itself
+      const int64_t c0 = (static_cast<int64_t>(strip) * SW + cc) * 8;
+      for (int64_t rr = tr; rr < rows; rr += rps) all.add(ld8<DT>(x, rr * c8 * 8 + c0));
+    }
+    all.across(SW);
+    if (t % kWave < SW) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) atomicMax(&smax[1][e * SW + cc], __float_as_uint(all.get(e)));
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  if (t < 8 * SCC) scale_out[b * SCC * 8 + t] = s_nan ? __builtin_nanf("") : 1.0f / inv_mine;
+  const unsigned int* const gm = smax[nrb > 1];
+  float iv[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) iv[e] = inv_scale(__uint_as_float(gm[e * SW + cc]), eps, kQmaxInt8);
+  if (rb == 0 && t < SW && col_ok) {
+    float* so = scale_out + (static_cast<int64_t>(strip) * SW + cc) * 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) so[e] = 1.0f / iv[e];
+  }
 
-  // Pass 2: multipliers of the thread's chunk-columns, then the cast.
-  float iv[CPT][8];
+  // Pass 2: the cast.
+  auto put = [&](const Raw8<DT>& v, int j) {
+    const int64_t left = (xe - j * xs) / elem_bytes<DT>();
+    const auto rq = __builtin_amdgcn_make_buffer_rsrc(qb + j * xs / elem_bytes<DT>(), 0,
+                                                      static_cast<int>(left > 0 ? left : 0),
+                                                      kBufDword3);
+    const uint2 c = cast8_cols<DT>(v, iv);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, u32x2{c.x, c.y}), rq, qv, 0,
+                                          CBQ_NT_STORES_NARROW ? kAuxNT : 0);
+  };
 #pragma unroll
-  for (int s = 0; s < CPT; ++s) {
-    if (ok2) {
-      ld8_pairs(inv64, C8, t + 1024 * s, iv[s]);
-    } else {
+  for (int k = 0; k < HS; ++k)
+    if (held0 + k < I) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) iv[s][e] = __builtin_nanf("");
+      for (int u = 0; u < U; ++u) put(r[k * U + u], (held0 + k) * U + u);
     }
-  }
-#pragma unroll
-  for (int k = 0; k < HS; ++k) {
-    const int64_t c0 = (held0 + k) * GS + cb;
-    const int64_t left = n8 - c0;
-    if (left > 0) {
-      const auto rs = rsrc(q + c0 * 8, (left < SB ? left : SB) * 8);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint2 c = cast8_cols<DT>(r[k * U + u], iv[u % CPT]);
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, u32x2{c.x, c.y}), rs,
-                                              u * kFusedBlock * 8 + qo, 0,
-                                              CBQ_NT_STORES_NARROW ? kAuxNT : 0);
-      }
-    }
-  }
-  const int64_t parked = held0 < LS ? held0 : LS;
-  for (int64_t i = 0; i < parked; ++i) {
+  const int parked = held0 < LS ? held0 : LS;
+  for (int i = 0; i < parked; ++i) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const u32x4* pk = park + (static_cast<int>(i) * U + u) * QW * kFusedBlock + t;
+      const u32x4* pk = park + (i * U + u) * QW * kFusedBlock + t;
       Raw8<DT> v;
       const u32x4 a = pk[0];
       v.a = make_uint4(a.x, a.y, a.z, a.w);
@@ -926,16 +909,15 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_cols_1pass(
         const u32x4 bb = pk[kFusedBlock];
         v.b = make_uint4(bb.x, bb.y, bb.z, bb.w);
       }
-      stg8(qw + (i * GS + u * kFusedBlock) * 8 + qo, cast8_cols<DT>(v, iv[u % CPT]));
+      put(v, i * U + u);
     }
   }
-  for (int64_t i = parked; i < held0; ++i) {
+  for (int i = parked; i < held0; ++i) {
     Raw8<DT> v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = ld8_at<DT>(xw + (i * GS + u * kFusedBlock) * EB, xo);
+    for (int u = 0; u < U; ++u) v[u] = load(i * U + u);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      stg8(qw + (i * GS + u * kFusedBlock) * 8 + qo, cast8_cols<DT>(v[u], iv[u % CPT]));
+    for (int u = 0; u < U; ++u) put(v[u], i * U + u);
   }
 }
 
@@ -2237,47 +2219,95 @@ ColGeom col_geom(int64_t rows, int64_t cols, bool vec) {
   return g;
 }
 
-// Grid of the one-launch column quant (k_quant_cols_1pass) for x of rows x
-// cols, or 0 when it does not apply: rows of 8192, 16384 or 32768 elements,
-// at least kColsMinElems elements, a power-of-two grid of at most one
-// workgroup per CU that splits the chunk-columns into slices of at most
-// kColsMaxSlice.
-int cols_1pass_grid(int64_t rows, int64_t cols) {
-  if (cols != 8192 && cols != 16384 && cols != 32768) return 0;
-  if (rows * cols < kColsMinElems) return 0;
-  int g = 1;
-  while (2 * g <= device_cus() && 2 * g <= kMaxFusedGrid) g *= 2;
-  const int64_t c8 = cols / 8;
-  if (c8 % g != 0 || c8 / g > kColsMaxSlice) return 0;
+// Geometry of the one-launch column quant (k_quant_cols_strip) for x of rows
+// x cols of elem_size bytes; strips == 0 when it does not apply (cols % 8 !=
+// 0, more strips than CUs, x above CBQ_COLS_1PASS_MAX_BYTES or, with an
+// exchange, below kStripMinBytes).
+//  * few rows: strips of 256 or 128 bytes per row with a single row block of
+//    at most 64 bytes per thread (128 for 2-byte types in 128-byte strips),
+//    no exchange. Kernels of a quant + dequant pass, bf16, against the
+//    column maxima + finalize + cast launches: [512, 4096] 15.8 -> 12.6 us,
+//    [100, 14336] 15.4 -> 12.3, [1024, 1024] 12.9 -> 12.5; fp32 quant [200,
+//    2000] 11.6 -> 7.3. Longer walks lose (fp32 [1000, 1000] as 8 chunks per
+//    thread 11.0 -> 17.5: 64 workgroups cannot stream 4 MB).
+//  * else strips of 64 chunks, or 32 or 16 where that leaves at least 6%
+//    fewer idle lanes in the last one (the whole row below 64 chunks), in as
+//    many row blocks as fill the CUs, each at least 32 KiB of x. [11008, 4096]
+//    70.8 -> 55.1 us, [8192, 8192] 77.4 -> 72.6 (the one-launch kernel this
+//    replaces took only rows of 8192, 16384 and 32768), [28672, 8192] 295.1
+//    -> 293.2, [262144, 64] 35.8 -> 26.2, [1024, 2048] 15.7 -> 14.9; below
+//    kStripMinBytes the exchange costs more than the two launches it saves
+//    ([2000, 512] 12.6 -> 13.9 us).
+constexpr int64_t kStripAloneBytes = 4 << 20, kStripMinBytes = 5 << 19;
+
+struct StripGeom {
+  int sl, strips, nrb;
+  int64_t RB;
+};
+
+StripGeom strip_geom(int64_t rows, int64_t cols, int elem_size) {
+  StripGeom g{0, 0, 0, 0};
+  const int64_t c8 = cols / 8, cus = std::min<int64_t>(device_cus(), kMaxFusedGrid);
+  if (cols % 8 != 0 || rows * cols * elem_size > CBQ_COLS_1PASS_MAX_BYTES) return g;
+  const int64_t bytes = rows * cols * elem_size;
+  const int narrow = elem_size == 4 ? 2 : 3;   // strips of 128 bytes per row
+  for (const int64_t slots : {4, 8})
+    for (int sl = slots == 4 ? narrow + 1 : narrow; sl >= narrow; --sl)
+      if ((rows << sl) * elem_size <= slots * 2 * kFusedBlock && bytes <= kStripAloneBytes &&
+          cdiv(c8, 1LL << sl) <= cus && (slots == 4 || elem_size == 2)) {
+        g = {sl, static_cast<int>(cdiv(c8, 1LL << sl)), 1, rows};
+        return g;
+      }
+  if (bytes < kStripMinBytes) return g;
+  int sl = kColsMaxSL;
+  while (sl > 0 && (1LL << (sl - 1)) >= c8) --sl;
+  if (sl == kColsMaxSL)
+    for (const int s2 : {5, 4})
+      if (cdiv(c8, 1LL << s2) * (1LL << s2) * 106 < cdiv(c8, 1LL << sl) * (1LL << sl) * 100) sl = s2;
+  const int64_t strips = cdiv(c8, 1LL << sl);
+  if (strips > cus) return g;
+  const int64_t min_rows = (elem_size == 4 ? 1 : 2) * (kFusedBlock >> sl);
+  const int64_t nrb = std::max<int64_t>(1, std::min(cus / strips, rows / min_rows));
+  const int64_t RB = cdiv(rows, nrb);
+  if ((RB + kFusedBlock * 4) * cols * elem_size >= (1LL << 31)) return g;
+  g.sl = sl;
+  g.strips = static_cast<int>(strips);
+  g.nrb = static_cast<int>(cdiv(rows, RB));
+  g.RB = RB;
   return g;
 }
 
-// True if one workgroup of k_quant_cols_1pass<DT, CPT> fits on a CU, so that
-// the whole grid is resident at once (cached per device and instantiation).
-template <int DT, int CPT>
-bool cols_1pass_fits() {
-  static int cached[64];   // 0 unknown, 1 fits, 2 does not
+// Bytes of partial maxima of that path (fp32 for fp32 input, else 16 bits).
+int64_t strip_part_bytes(const StripGeom& g, int elem_size) {
+  return static_cast<int64_t>(g.strips) * g.nrb * (8LL << g.sl) * elem_size;
+}
+
+// True if one workgroup of k_quant_cols_strip<DT> fits on a CU, so that the
+// whole grid is resident at once (cached per device and instantiation).
+template <int DT>
+bool cols_strip_fits() {
+  static std::atomic<int> cached[64];   // 0 unknown, 1 fits, 2 does not
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-  if (cached[dev] == 0) {
+  int c = cached[dev].load(std::memory_order_relaxed);
+  if (c == 0) {
     int nb = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &nb, reinterpret_cast<const void*>(&k_quant_cols_1pass<DT, CPT>), kFusedBlock, 0);
-    cached[dev] = (e == hipSuccess && nb >= 1) ? 1 : 2;
+        &nb, reinterpret_cast<const void*>(&k_quant_cols_strip<DT>), kFusedBlock, 0);
+    c = (e == hipSuccess && nb >= 1) ? 1 : 2;
+    cached[dev].store(c, std::memory_order_relaxed);
   }
-  return cached[dev] == 1;
+  return c == 1;
 }
 
 size_t col_ws_bytes(int64_t rows, int64_t cols) {
   // The byte count does not depend on the vector path: nrb is computed for
   // the smaller (vector) column-block count, which never yields fewer row
-  // blocks than the scalar path does. The one-launch path needs one [cols]
-  // row of partial maxima per workgroup plus the [cols] multipliers.
+  // blocks than the scalar path does. The one-launch path's partial maxima
+  // fit the same room (fewer, 64-chunk-wide blocks) and are used only then.
   const ColGeom gv = col_geom(rows, cols, true);
   const ColGeom gs = col_geom(rows, cols, false);
-  int64_t nrb = gv.nrb > gs.nrb ? gv.nrb : gs.nrb;
-  const int64_t g1 = cols_1pass_grid(rows, cols);
-  if (g1 > nrb) nrb = g1;
+  const int64_t nrb = gv.nrb > gs.nrb ? gv.nrb : gs.nrb;
   return CBQ_WS_CTRL_BYTES + static_cast<size_t>(nrb) * cols * 4 + static_cast<size_t>(cols) * 4;
 }
 
@@ -2300,26 +2330,17 @@ template <int DT>
 int cols_quant_t(const void* x, int64_t rows, int64_t cols, int64_t inner, float eps, void* ws,
                  int8_t* q, float* scale, hipStream_t s, const char* what) {
   const bool vec = (cols % 8 == 0) && aligned(x, 16) && aligned(q, 8);
-  if (vec && inner == 1 && rows * cols * elem_bytes<DT>() <= CBQ_COLS_1PASS_MAX_BYTES) {
-    const int g1 = cols_1pass_grid(rows, cols);
-    const int cpt = static_cast<int>(cols / 8192);
-    if (g1 > 0 && (cpt == 1   ? cols_1pass_fits<DT, 1>()
-                   : cpt == 2 ? cols_1pass_fits<DT, 2>()
-                              : cols_1pass_fits<DT, 4>())) {
+  if (vec && inner == 1) {
+    const StripGeom sg = strip_geom(rows, cols, elem_bytes<DT>());
+    if (sg.strips > 0 && CBQ_WS_CTRL_BYTES + strip_part_bytes(sg, elem_bytes<DT>()) <=
+                             static_cast<int64_t>(col_ws_bytes(rows, cols)) &&
+        cols_strip_fits<DT>()) {
       char* ctl = static_cast<char*>(ws);
-      float* part = reinterpret_cast<float*>(ctl + CBQ_WS_CTRL_BYTES);
-      float* invs = part + static_cast<int64_t>(g1) * cols;
-      const int64_t n8 = rows * cols / 8;
-      const dim3 grid(static_cast<unsigned>(g1)), blk(kFusedBlock);
-      if (cpt == 1)
-        k_quant_cols_1pass<DT, 1><<<grid, blk, 0, s>>>(x, n8, eps, q, scale, ctl, part, invs,
-                                                       fused_spin_limit());
-      else if (cpt == 2)
-        k_quant_cols_1pass<DT, 2><<<grid, blk, 0, s>>>(x, n8, eps, q, scale, ctl, part, invs,
-                                                       fused_spin_limit());
-      else
-        k_quant_cols_1pass<DT, 4><<<grid, blk, 0, s>>>(x, n8, eps, q, scale, ctl, part, invs,
-                                                       fused_spin_limit());
+      k_quant_cols_strip<DT><<<dim3(static_cast<unsigned>(sg.strips * sg.nrb)), dim3(kFusedBlock), 0,
+                               s>>>(x, rows, static_cast<int>(cols / 8), sg.sl, sg.strips, sg.nrb,
+                                    sg.RB, eps, q, scale, ctl,
+                                    reinterpret_cast<unsigned long long*>(ctl + CBQ_WS_CTRL_BYTES),
+                                    std::min(fused_spin_limit(), kColsSpinLimit));
       return launch_status(what);
     }
   }

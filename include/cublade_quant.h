@@ -57,8 +57,11 @@ enum { CBQ_OK = 0, CBQ_EINVAL = 1, CBQ_ELAUNCH = 2 };
  * call writes a NaN scale whenever any of its codes is not exact (FP8 codes
  * NaN, INT8 codes 0 there); a scale that is not NaN comes with every code
  * exact. The next call on the workspace is exact again, with no reset; the
- * status word stays 1 until cbq_tensor_quant_status_clear. The other entry
- * points leave the control block alone. The rest is per-call scratch. One
+ * status word stays 1 until cbq_tensor_quant_status_clear. Per-column quant
+ * (cbq_quant_int8_channel, axis 1) uses the block the same way, but a
+ * workgroup that gives up there takes the maxima of its columns from x itself:
+ * its results are exact either way, only the status word tells. The other
+ * entry points leave the control block alone. The rest is per-call scratch. One
  * workspace serves one stream at a time: calls that overlap in time must not
  * share it. */
 #define CBQ_WS_CTRL_BYTES 16384

@@ -1,19 +1,16 @@
 """The one-launch per-column (axis 1) quant, against the oracle, bit for bit.
 
-k_quant_cols_1pass takes rows of 8192, 16384 or 32768 elements (x of 2^22
-elements up to 480 MiB, 16-byte aligned; larger x takes the two-pass path,
-which the full config-3 test covers): the per-tensor one-launch step layout
-(grid-wide steps of 2^23 elements on 256 CUs; the last HS steps of each
-thread held in registers, the first LS streamed ones parked in LDS, the
-others read again after the exchange) with per-column running maxima, then
-two grid-wide exchanges (partial column maxima; the multipliers of each
-workgroup's slice of columns). Random data puts each column's maximum in a
-random row, so across the columns every part of the layout holds some
-column's maximum; explicit outlier columns are added in the parked, re-read,
-first held and last held parts. Codes, scales and the dequantized outputs are
+Rows of 8192, 16384 and 32768 elements and x of 2^22 elements up to 480 MiB
+(k_quant_cols_strip; larger x takes the two-pass path, which the full config-3
+test covers). Random data puts each column's maximum in a random row, so across
+the columns every part of a block (held in registers, parked in LDS, read again
+after the exchange) holds some column's maximum; explicit outlier columns are
+added in row ranges spread over x. Codes, scales and the dequantized outputs are
 compared bit for bit with the oracle, through the public API
 (quantize_tensor(..., mode="channel", ch_axis=1)) and through the C ABI.
 
+The row ranges are those of grid-wide steps of 2^23 elements on 256 CUs, of
+which the last HS and the first LS stay on chip:
 Sizes (hold steps HS / parked LS per row length and dtype): one partial step
 (fewer workgroups with data than CUs), held only, held + parked, and held +
 parked + re-read with a ragged last step, for each row length; fp32 as well.
