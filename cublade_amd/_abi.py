@@ -24,6 +24,7 @@ SOURCES = [
     CSRC / "cbq_quant.hip",
     CSRC / "cbq_dequant.hip",
     CSRC / "cbq_w8a16.hip",
+    CSRC / "cbq_w8a16_f32.hip",
     CSRC / "cbq_gemm.hip",
 ]
 

@@ -59,6 +59,7 @@
 #include "cbq_device.h"
 #include "cbq_host.h"
 #include "cbq_lds_dma.h"
+#include "cbq_w8a16_f32.h"
 
 namespace cbq {
 namespace {
@@ -136,7 +137,6 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   int splits, split_steps;  // split-K: number of k-ranges, 64-k steps per range
   int full_tiles;           // split-K: tiles [0, full_tiles) run whole, the rest split
-  const uint16_t* x2;       // k_gemm_dma<.., PLANES>: the second x plane (splits >= splits / 2)
 };
 
 // Workgroup b of n goes to XCD b % 8; renumbered so that each XCD takes a
@@ -497,7 +497,7 @@ __device__ __forceinline__ void outlier_mfma(const uint8_t* so, int wm, int wn, 
 // the others split the remaining tiles over `splits` k-ranges, workgroup
 // full_tiles + b covering tail tile b % rest of k-range b / rest (after the
 // XCD renumbering, so the workgroups of one XCD share a k-range of x).
-template <int ACT, bool SPLIT, int TM, bool PLANES = false, int TNW = kDmaTN, int WM = 2>
+template <int ACT, bool SPLIT, int TM, int TNW = kDmaTN, int WM = 2>
 __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
   constexpr int WN = 8 / WM;   // waves along N
   constexpr int BM = WM * 32 * TM, BN = WN * 32 * TNW, BK = 64, NS = 3;
@@ -545,12 +545,8 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
     decode_tile(blockIdx.x, a, tm, tn);
   }
   const int m0 = tm * BM, n0 = tn * BN;
-  // PLANES: splits = 2 KS, split s runs k-range s % KS of x plane s / KS
-  const int ks = PLANES ? a.splits / 2 : 1;
-  const int krange = PLANES ? split % ks : split;
-  const int kb = partial ? krange * a.split_steps : 0;   // first 64-k step
+  const int kb = partial ? split * a.split_steps : 0;   // first 64-k step
   const int nk = partial ? min(a.split_steps, a.K / BK - kb) : a.K / BK;
-  const uint16_t* const xsrc = (PLANES && split >= ks) ? a.x2 : a.x;
   const uint32_t sbase = __builtin_amdgcn_readfirstlane(lds_addr(smem));
 
   // Per-lane DMA source offsets (bytes from the k0 column of the tile). x
@@ -576,7 +572,7 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
   // DMA instruction u (0..XL+WL-1) of tile t into `stage`.
   auto issue_one = [&](int t, int stage, int u) {
     if (u < XL)
-      lds_dma16(xo[u], uniform_ptr(xsrc + (kb + t) * BK), sbase + stage * SB + wave * 1024 + u * 8192);
+      lds_dma16(xo[u], uniform_ptr(a.x + (kb + t) * BK), sbase + stage * SB + wave * 1024 + u * 8192);
     else
       lds_dma16(wo[u - XL], uniform_ptr(a.wq + (kb + t) * BK),
                 sbase + stage * SB + XB + wave * 1024 + (u - XL) * 8192);
@@ -714,7 +710,7 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
 #pragma unroll
   for (int t = 0; t < NS; ++t)
     if (t < nk) issue(t, t);
-  if (!PLANES && tid < 256) {   // the two-plane launches carry no scales
+  if (tid < 256) {
     const int n = n0 + tid;
     const int nc = min(n, a.N - 1);
     const float sv = act_to_f32<ACT>(a.scales[nc]);
@@ -865,7 +861,7 @@ void launch_gemm_dma128(GemmArgs a, hipStream_t s) {
   a.tiles_m = static_cast<int>(cdiv(a.M, 128));
   a.tiles_n = static_cast<int>(cdiv(a.N, 128));
   const unsigned grid = static_cast<unsigned>(a.tiles_m) * a.tiles_n;
-  k_gemm_dma<ACT, false, 2, false, 1, 2><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
+  k_gemm_dma<ACT, false, 2, 1, 2><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
 }
 
 // Split-K finish: each thread takes two partial f4 of a tail tile, kBlock
@@ -1036,91 +1032,6 @@ __global__ __launch_bounds__(kBlock) void k_splitk_reduce(GemmArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (nb + r < a.N) dst[r] = out1<ACT>(v[u][r]);
-    }
-  }
-}
-
-// fp32 activations on the matrix cores. The weights are int8, exact in
-// bf16, so x . w = hi . w + lo . w + r . w with hi = x truncated to bf16
-// (never rounds up to inf), lo = bf16(x - hi) (x - hi is exact: the low 16
-// bits of x's significand) and |r| <= 2^-16 |x|: each bf16 x int8 product is
-// exact in the fp32 accumulators, and x keeps 16 significant bits (the
-// reference's fp32 Triton dot runs at TF32 precision, 11 bits). Non-finite x:
-// hi carries it (NaN canonical), lo = 0. k_f32_planes writes the two planes;
-// k_gemm_dma<BF16, true, TM, true> then runs every tile once per plane and
-// k-range (KS ranges per plane: 1, or up to 8 for M <= 64) into fp32 partial
-// tiles, and k_planes_reduce adds them in order and applies the fp32 scale
-// and bias.
-__global__ __launch_bounds__(kBlock) void k_f32_planes(const float* __restrict__ x, int64_t n4,
-                                                     uint16_t* __restrict__ xh,
-                                                     uint16_t* __restrict__ xl) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= n4) return;
-  const f4 v = reinterpret_cast<const f4*>(x)[i];
-  uint32_t hb[4];
-  float lo[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const uint32_t b = __float_as_uint(v[r]);
-    const bool fin = (b & 0x7f800000u) != 0x7f800000u;
-    const bool nan = !fin && (b & 0x007fffffu) != 0;
-    hb[r] = nan ? 0x7fc0u : (b >> 16);
-    lo[r] = fin ? v[r] - __uint_as_float(hb[r] << 16) : 0.0f;
-  }
-  reinterpret_cast<uint2*>(xh)[i] = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
-  reinterpret_cast<uint2*>(xl)[i] =
-      make_uint2(pack2_out<kBF16>(lo[0], lo[1]), pack2_out<kBF16>(lo[2], lo[3]));
-}
-
-// The 2 KS partial planes of every tile (layout as in k_splitk_reduce, all
-// tiles split: the k-ranges of x plane hi, then those of plane lo), summed in
-// that order -> y = fp32(sum * s[n] + bias[n]). Each thread takes two
-// partial f4, kBlock apart.
-template <int TM>
-__global__ __launch_bounds__(kBlock) void k_planes_reduce(GemmArgs a, const float* __restrict__ sc,
-                                                          const float* __restrict__ bias,
-                                                          float* __restrict__ y) {
-  constexpr int kWaveF4 = kDmaTN * TM * 4 * 64;
-  constexpr int kTileF4 = 8 * kWaveF4;
-  static_assert(kTileF4 % (kBlock * 2) == 0, "a thread's f4 share a tile");
-  const int tiles = a.tiles_m * a.tiles_n;
-  const int64_t per_plane = static_cast<int64_t>(tiles) * kTileF4;
-  const int64_t idx0 = static_cast<int64_t>(blockIdx.x) * (kBlock * 2) + threadIdx.x;
-  if (idx0 >= per_plane) return;
-  const f4* src = reinterpret_cast<const f4*>(a.part) + idx0;
-  f4 sum[2] = {src[0], src[kBlock]};
-#pragma unroll 4
-  for (int p = 1; p < a.splits; ++p) {
-    const f4* q = src + p * per_plane;
-    sum[0] += q[0];
-    sum[1] += q[kBlock];
-  }
-  int tm, tn;
-  group_tile(static_cast<int>(idx0 / kTileF4), a, tm, tn);
-  const bool vec = (a.N % 4) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int w = static_cast<int>((idx0 + u * kBlock) % kWaveF4);
-    const int lane = w & 63, q = (w >> 6) & 3, j = (w >> 8) % TM, i = (w >> 8) / TM;
-    const int wave = static_cast<int>(((idx0 + u * kBlock) / kWaveF4) & 7);
-    const int m = tm * 64 * TM + (wave & 1) * 32 * TM + j * 32 + (lane & 31);
-    const int nb = tn * 256 + (wave >> 1) * 64 + i * 32 + 8 * q + 4 * (lane >> 5);
-    if (m >= a.M || nb >= a.N) continue;
-    f4 v;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = nb + r < a.N ? sum[u][r] * sc[nb + r] : 0.0f;
-    if (bias) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (nb + r < a.N) v[r] += bias[nb + r];
-    }
-    float* dst = y + static_cast<int64_t>(m) * a.N + nb;
-    if (vec && nb + 3 < a.N) {
-      *reinterpret_cast<f4*>(dst) = v;
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (nb + r < a.N) dst[r] = v[r];
     }
   }
 }
@@ -1964,150 +1875,6 @@ int64_t general_split_bytes(int64_t M, int64_t N, int64_t K) {
   return sp > 1 ? static_cast<int64_t>(sp) * M * N * 4 : 0;
 }
 
-// Two-plane fp32 path (see k_f32_planes): no outlier columns, the DMA
-// kernel's shape limits, and for M <= 64 a weight of at least 8 MB (below
-// that the general kernel's single launch is as fast). The x-tile height
-// with the fewest modelled step units over both planes' workgroups: rounds
-// of workgroups on the CUs times the full-occupancy cost of a 64-k step
-// (dma_plan's model: 1.12 / 1.46 / 1.85 us for 128 / 192 / 256-row tiles).
-// For M <= 64 (one row of 128-row tiles) K is also split into KS ranges, so
-// that the 2 KS planes' workgroups fill the CUs (at most 8 ranges of at
-// least four 64-k steps): fp32 x at M = 16, N = 11008, K = 4096 takes two
-// ranges, 172 workgroups.
-bool planes_ok(int64_t M, int64_t N, int64_t K, int64_t n_out) {
-  return n_out == 0 && dma_ok(M, N, K) && 2 * cdiv(M, 128) * cdiv(N, 256) < (1LL << 30) &&
-         (M > 64 || N * K >= (8LL << 20));
-}
-
-int planes_tm(int64_t M, int64_t N) {
-  const int64_t cus = device_cus();
-  const double cost[5] = {0.0, 0.0, 1.12, 1.46, 1.85};
-  int best_tm = 4;
-  double best = 1e300;
-  for (int tm = 2; tm <= 4; ++tm) {
-    const int64_t wgs = 2 * cdiv(M, static_cast<int64_t>(64 * tm)) * cdiv(N, static_cast<int64_t>(256));
-    const double t = static_cast<double>(cdiv(wgs, cus)) * cost[tm];
-    if (t < best - 1e-9) {
-      best = t;
-      best_tm = tm;
-    }
-  }
-  return best_tm;
-}
-
-struct PlanesPlan {
-  int tm, ks, steps;   // x-tile height / 64, k-ranges per plane, 64-k steps per range
-};
-
-PlanesPlan planes_plan(int64_t M, int64_t N, int64_t K) {
-  const int tm = planes_tm(M, N);
-  const int64_t tiles = cdiv(M, static_cast<int64_t>(64 * tm)) * cdiv(N, static_cast<int64_t>(256));
-  const int64_t nk = K / 64;
-  int64_t ks = 1;
-  if (M <= 64) ks = std::max<int64_t>(1, std::min<int64_t>({device_cus() / (2 * tiles), 8, nk / 4}));
-  const int64_t steps = cdiv(nk, ks);
-  return {tm, static_cast<int>(cdiv(nk, steps)), static_cast<int>(steps)};   // no empty ranges
-}
-
-// Bytes after the control block: the two bf16 planes (each 256-byte
-// aligned), then the fp32 partial tiles of every plane and k-range.
-int64_t planes_x_bytes(int64_t M, int64_t K) { return cdiv(M * K * 2, static_cast<int64_t>(256)) * 256; }
-
-int64_t planes_bytes(int64_t M, int64_t N, int64_t K) {
-  const PlanesPlan p = planes_plan(M, N, K);
-  const int64_t tiles = cdiv(M, static_cast<int64_t>(64 * p.tm)) * cdiv(N, static_cast<int64_t>(256));
-  return 2 * planes_x_bytes(M, K) + tiles * 2 * p.ks * (64 * p.tm) * 256 * 4;
-}
-
-// Workspace cap of the two-plane path: M is processed in chunks of rows
-// (multiples of 256, one after the other on the stream, reusing the
-// workspace) whose planes and partial tiles fit kPlanesMaxBytes (at M = 4096,
-// N = 11008, K = 4096 one launch would need 428 MB: two chunks of 2560 and
-// 1536 rows). A remainder of at most 64 rows joins the chunk before it, so
-// that every chunk keeps the plan of M > 64; chunks of 256 rows that alone
-// exceed the cap (very wide weights) are taken as they are.
-constexpr int64_t kPlanesMaxBytes = int64_t(256) << 20;
-
-int64_t planes_chunk_rows(int64_t M, int64_t N, int64_t K) {
-  if (planes_bytes(M, N, K) <= kPlanesMaxBytes) return M;
-  int64_t mc = 256;
-  while (mc + 256 < M && planes_bytes(mc + 256, N, K) <= kPlanesMaxBytes) mc += 256;
-  return mc;
-}
-
-// Rows of the chunk starting at m0.
-int64_t planes_chunk_at(int64_t m0, int64_t M, int64_t mc) {
-  const int64_t left = M - m0;
-  return left <= mc + 64 ? left : mc;
-}
-
-// Workspace of the two-plane path: the most any of its chunks needs (the
-// chunks of w8a16_f32_planes, walked the same way).
-int64_t planes_ws_bytes(int64_t M, int64_t N, int64_t K) {
-  const int64_t mc = planes_chunk_rows(M, N, K);
-  int64_t most = 0;
-  for (int64_t m0 = 0; m0 < M;) {
-    const int64_t mr = planes_chunk_at(m0, M, mc);
-    most = std::max(most, planes_bytes(mr, N, K));
-    m0 += mr;
-  }
-  return most;
-}
-
-template <int TM>
-void launch_planes(GemmArgs a, const PlanesPlan& p, const float* sc, const float* bias, float* y,
-                   hipStream_t s) {
-  a.tiles_m = static_cast<int>(cdiv(a.M, 64 * TM));
-  a.tiles_n = static_cast<int>(cdiv(a.N, 256));
-  a.full_tiles = 0;
-  a.splits = 2 * p.ks;
-  a.split_steps = p.steps;
-  const int tiles = a.tiles_m * a.tiles_n;
-  k_gemm_dma<kBF16, true, TM, true><<<dim3(static_cast<unsigned>(a.splits * tiles)),
-                                      dim3(kDmaThreads), 0, s>>>(a);
-  const int64_t n4 = static_cast<int64_t>(tiles) * 8 * kDmaTN * TM * 4 * 64;
-  k_planes_reduce<TM><<<dim3(static_cast<unsigned>(cdiv(n4, kBlock * 2))), dim3(kBlock), 0, s>>>(
-      a, sc, bias, y);
-}
-
-// The two-plane path when it applies (returns its status), else -1.
-int w8a16_f32_planes(const void* x, const int8_t* wq, const void* scales, const void* bias,
-                     int64_t n_out, int64_t M, int64_t N, int64_t K, void* ws, size_t ws_bytes,
-                     void* y, hipStream_t s) {
-  if (!planes_ok(M, N, K, n_out) || !ws || !aligned(x, 16) || !aligned(wq, 16) ||
-      ws_bytes < static_cast<size_t>(CBQ_WS_CTRL_BYTES + planes_ws_bytes(M, N, K)))
-    return -1;
-  const int64_t mc = planes_chunk_rows(M, N, K);
-  for (int64_t m0 = 0; m0 < M;) {
-    const int64_t mr = planes_chunk_at(m0, M, mc);
-    uint8_t* base = static_cast<uint8_t*>(ws) + CBQ_WS_CTRL_BYTES;
-    uint16_t* xh = reinterpret_cast<uint16_t*>(base);
-    uint16_t* xl = reinterpret_cast<uint16_t*>(base + planes_x_bytes(mr, K));
-    const int64_t n4 = mr * K / 4;   // K % 64 == 0
-    k_f32_planes<<<dim3(static_cast<unsigned>(cdiv(n4, static_cast<int64_t>(kBlock)))),
-                   dim3(kBlock), 0, s>>>(static_cast<const float*>(x) + m0 * K, n4, xh, xl);
-    GemmArgs a{};
-    a.x = xh;
-    a.x2 = xl;
-    a.wq = wq;
-    a.part = reinterpret_cast<float*>(base + 2 * planes_x_bytes(mr, K));
-    a.M = static_cast<int>(mr);
-    a.N = static_cast<int>(N);
-    a.K = static_cast<int>(K);
-    const float* sc = static_cast<const float*>(scales);
-    const float* bs = static_cast<const float*>(bias);
-    float* yo = static_cast<float*>(y) + m0 * N;
-    const PlanesPlan p = planes_plan(mr, N, K);
-    switch (p.tm) {
-      case 2: launch_planes<2>(a, p, sc, bs, yo, s); break;
-      case 3: launch_planes<3>(a, p, sc, bs, yo, s); break;
-      default: launch_planes<4>(a, p, sc, bs, yo, s); break;
-    }
-    m0 += mr;
-  }
-  return launch_status("cbq_w8a16_linear");
-}
-
 template <int ACT>
 int w8a16_general(const void* x, const int8_t* wq, const void* scales, const void* bias,
                   const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N,
@@ -2196,8 +1963,8 @@ extern "C" size_t cbq_w8a16_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t n_
   const bool mfma = (act_dtype == kF16 || act_dtype == kBF16) && K % 16 == 0;
   const int64_t bytes =
       mfma ? splitk_bytes(M, N, split_plan(M, N, K))
-      : (act_dtype == kF32 && planes_ok(M, N, K, n_out))
-          ? std::max(planes_ws_bytes(M, N, K), general_split_bytes(M, N, K))
+      : (act_dtype == kF32 && f32lin::applies(M, N, K, n_out))
+          ? std::max(f32lin::ws_bytes(M, N, K), general_split_bytes(M, N, K))
           : general_split_bytes(M, N, K);
   return CBQ_WS_CTRL_BYTES + static_cast<size_t>(bytes);
 }
@@ -2231,9 +1998,12 @@ extern "C" int cbq_w8a16_linear(const void* x, int act_dtype, const int8_t* wq,
                                                      N, K, nullptr, 0, y, s);
   }
   if (act_dtype == kF32) {
-    const int rc = w8a16_f32_planes(x, wq, scales, bias, n_out, M, N, K, ws, ws_bytes, y,
-                                    as_stream(stream));
-    if (rc >= 0) return rc;
+    if (f32lin::applies(M, N, K, n_out) && ws && aligned(x, 16) && aligned(wq, 16) &&
+        ws_bytes >= static_cast<size_t>(CBQ_WS_CTRL_BYTES + f32lin::ws_bytes(M, N, K)))
+      return f32lin::run(static_cast<const float*>(x), wq, static_cast<const float*>(scales),
+                         static_cast<const float*>(bias), M, N, K,
+                         static_cast<uint8_t*>(ws) + CBQ_WS_CTRL_BYTES, static_cast<float*>(y),
+                         as_stream(stream), what);
     return w8a16_general<kF32>(x, wq, scales, bias, outlier_cols, n_out, w_out, M, N, K, ws,
                               ws_bytes, y, as_stream(stream));
   }

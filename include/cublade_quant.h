@@ -250,15 +250,13 @@ int cbq_dequant_int8_group_nd(const int8_t* q, const float* scale,
  * last wave of output tiles is short, the fp32 partial tiles of that wave
  * (ranges x tail tiles x 256 / 192 / 128 KiB for tiles of 256 / 192 / 128 x
  * 256; at most 16 ranges and at most one partial tile per CU, i.e. <= 64 MiB
- * on MI355X; the same with outlier columns), else nothing. CBQ_F32 on the matrix-core path (see
- * cbq_w8a16_linear): two bf16 planes of x (4 M K bytes) and the fp32
- * partial tiles of both planes (8 bytes per output of the padded tiles; for
- * M <= 64 times the k-ranges per plane, at most 8: 32 MB at M = 16, N = 4096,
- * K = 11008), capped at 256 MiB: a larger M runs in chunks of rows
- * (multiples of 256, one after another, reusing the workspace), so the size
- * is that of the largest chunk (M = 4096, N = 11008, K = 4096: chunks of 2560
- * and 1536 rows, 241 MB instead of 428 MB; chunks of 256 rows that alone
- * exceed the cap are used as they are). Other CBQ_F32
+ * on MI355X; the same with outlier columns), else nothing. CBQ_F32 on the
+ * matrix-core path (see cbq_w8a16_linear): three int8 digit planes of x
+ * (3 M K bytes; the size is never below 4 M K), 520 bytes per row of scales
+ * and spike lists (per k-range above K = 16384) and, when K is split, 4 bytes
+ * per output and k-range (at most 16 and at most one tile per CU). A larger M
+ * runs in chunks of rows (multiples of 256, one after another, reusing the
+ * workspace) whose 4 M K bytes stay below 256 MiB. Other CBQ_F32
  * shapes and K % 16 != 0 (general kernel): fp32 partial sums, up to 16 x M x
  * N x 4 bytes when its tiles give fewer than two workgroups per CU. The
  * reference allocates its temporaries inside the forward (linear.py:105-131). */
@@ -276,10 +274,10 @@ size_t cbq_w8a16_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t n_out, int ac
  * x: [M,K] and y: [M,N] in act_dtype, row-major. CBQ_F16 / CBQ_BF16 run
  * on MFMA. CBQ_F32 (the reference's fp32 Triton path, TF32 precision on its
  * hardware) with K % 64 == 0, no outlier columns, M > 64 or a weight of at
- * least 8 MB, and a workspace of cbq_w8a16_ws_bytes also runs on MFMA (for
- * M <= 64 with K split into up to 8 ranges): x is split into two bf16 planes
- * (hi = x truncated, lo = bf16(x - hi): 16 significant bits of x, exact
- * products with the int8 weights, fp32 accumulation); other CBQ_F32 calls,
+ * least 8 MB, and a workspace of cbq_w8a16_ws_bytes also runs on MFMA: each
+ * row of x as 24-bit fixed-point numbers against its largest magnitude, three
+ * int8 digits multiplied exactly (elements above 128 times the row's mean
+ * magnitude and non-finite ones are added in fp32); other CBQ_F32 calls,
  * K % 16 != 0 and unaligned operands run a tiled fp32-FMA kernel. K == 0
  * gives y = bias (or 0); x and wq may then be null.
  * wq: int8 [N,K] row-major; its outlier columns hold 0.

@@ -3,7 +3,7 @@ against the oracle's exact-accumulation W8A16 (float64) and the golden
 vectors. Gate (north star): rtol 1e-2 / atol 1e-2.
 
 Covers the MFMA path (fp16 / bf16, M / N / K tails), fp32 activations on the
-matrix cores as two bf16 planes (M > 64, K % 64 == 0), the general path (other
+matrix cores as int8 digits (M > 64, K % 64 == 0), the general path (other
 fp32 shapes, K not a multiple of 16, unaligned activations), bias, the
 outlier side-GEMM, quantize_model on an MLP, state_dict round trips (own and
 reference compact layout) and the BASELINE config-5 shapes (row subsets
@@ -163,14 +163,12 @@ def test_general_path_fp32_tiles(M, K, N):
                                    (40, 2048, 4160), (64, 11008, 1024), (5160, 4096, 11008)])
 def test_fp32_two_plane_path(M, K, N):
     """fp32 activations with K % 64 == 0, no outlier columns and M > 64 (or
-    M <= 64 with a weight of at least 8 MB, then K also split into up to 8
-    ranges per plane) run on the matrix cores as two bf16 planes of x (hi
-    truncated, lo = bf16(x - hi)) against the int8 weights; M = 5160 at
-    N = 11008 exceeds the path's 256 MiB workspace cap and runs as chunks of
-    2560 and 2600 rows (the 40-row remainder joins the last chunk). Sampled rows
+    M <= 64 with a weight of at least 8 MB; K may be split into
+    ranges) run on the matrix cores as int8 digits of x against the int8
+    weights. Sampled rows
     against the oracle; the whole output against a float64 product within
-    2^-14 of sum_k |x w s| (x keeps 16 significant bits; dropping the lo plane
-    would leave only 8); with outlier columns the VALU kernel runs, also
+    2^-14 of sum_k |x w s| (one digit less would leave 16 bits against the
+    row's largest element); with outlier columns the VALU kernel runs, also
     against the oracle."""
     from cublade_amd import _abi
     assert _abi.lib().cbq_w8a16_ws_bytes(M, N, K, 0, _abi.DTYPE_CODE[torch.float32]) > \
@@ -189,7 +187,7 @@ def test_fp32_two_plane_path(M, K, N):
 
 
 def test_fp32_two_plane_path_special_values():
-    """NaN, +-inf and huge finite activations: the two-plane path and the VALU
+    """NaN, +-inf and huge finite activations: the matrix-core path and the VALU
     kernel (forced by a control-block-only workspace) give the same NaN and
     inf pattern and close finite values."""
     from cublade_amd import _abi
