@@ -442,8 +442,17 @@ int64_t chunk_bytes(int64_t M, int64_t N, int64_t K) {
   const F32Plan p = f32_plan(M, N, K);
   const int64_t need = align256(3 * M * K) + align256(f32_segs(K, p) * M * (2 + kMaxSpikes) * 4) +
                        (p.splits > 1 ? p.splits * M * N * 4 : 0);
-  // never below the size of x, which this path has always asked for
-  return std::max(need, align256(4 * M * K + 1));
+  // The size never falls below what earlier versions of the library asked for,
+  // so that workspaces shared with a caller's other buffers keep their layout:
+  // two 16-bit planes of x and, at M <= 64, fp32 tiles of 128 x 256 for each
+  // plane and k-range (as many ranges as fill the CUs, at most 8).
+  int64_t before = 2 * align256(2 * M * K) + 256;
+  if (M <= 64) {
+    const int64_t tiles = cdiv(N, 256LL), nk = K / 64;
+    const int64_t ks = std::max<int64_t>(1, std::min<int64_t>({device_cus() / (2 * tiles), 8, nk / 4}));
+    before += tiles * 2 * cdiv(nk, cdiv(nk, ks)) * 128 * 256 * 4 - 256;
+  }
+  return std::max(need, before);
 }
 
 template <int TN, int WM>
