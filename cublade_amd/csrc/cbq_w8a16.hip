@@ -29,7 +29,7 @@
 // contiguous run of tiles, and tiles run in groups of 8 m-tiles, so the
 // workgroups resident on one XCD share activation and weight k-slices in L2.
 //
-// k_gemm_dma<ACT, SPLIT, TM> (M > 64, K % 64 == 0): 64 TM x 256 tiles (TM =
+// k_gemm_dma<ACT, SPLIT, TM> (M > 64, K % 16 == 0): 64 TM x 256 tiles (TM =
 // 4, 3, 2) of v_mfma_f32_32x32x16 fed by LDS DMA, 8 waves (two per SIMD),
 // int8 weights widened after the fragment read, explicitly scheduled k-steps
 // (see the kernel's comment). With SPLIT, the tiles of a short last wave run
@@ -409,8 +409,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm(GemmArgs a) {
 // (0..3) takes k [32 h + 8 s, 32 h + 8 s + 8) from both operands, so A and B
 // see the same k permutation and the products are unchanged.
 //
-// Requirements (checked on the host): K % 64 == 0, x and wq 16-byte aligned,
+// Requirements (checked on the host): K % 16 == 0, x and wq 16-byte aligned,
 // M * K * 2 and N * K below 2^32 (32-bit per-lane offsets from a scalar base).
+// K % 64 != 0 ends in a short step (see issue_short).
 // Rows past M or N are clamped to the last row; their products land in
 // outputs that are never stored.
 
@@ -497,7 +498,7 @@ __device__ __forceinline__ void outlier_mfma(const uint8_t* so, int wm, int wn, 
 // the others split the remaining tiles over `splits` k-ranges, workgroup
 // full_tiles + b covering tail tile b % rest of k-range b / rest (after the
 // XCD renumbering, so the workgroups of one XCD share a k-range of x).
-template <int ACT, bool SPLIT, int TM, int TNW = kDmaTN, int WM = 2>
+template <int ACT, bool SPLIT, int TM, int TNW = kDmaTN, int WM = 2, bool SHORT = false>
 __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
   constexpr int WN = 8 / WM;   // waves along N
   constexpr int BM = WM * 32 * TM, BN = WN * 32 * TNW, BK = 64, NS = 3;
@@ -546,7 +547,12 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
   }
   const int m0 = tm * BM, n0 = tn * BN;
   const int kb = partial ? split * a.split_steps : 0;   // first 64-k step
-  const int nk = partial ? min(a.split_steps, a.K / BK - kb) : a.K / BK;
+  // SHORT: K % 64 != 0, the last step is short (see issue_short). An instance
+  // of its own: the extra code costs the others 1-5% ([1000, 1024] x [1024,
+  // 1024] 13.7 -> 14.5 us).
+  const int nkt = SHORT ? a.K / BK + 1 : a.K / BK;
+  const int nk = partial ? min(a.split_steps, nkt - kb) : nkt;
+  const int nkf = SHORT ? min(nk, a.K / BK - kb) : nk;   // whole steps (nk or nk - 1)
   const uint32_t sbase = __builtin_amdgcn_readfirstlane(lds_addr(smem));
 
   // Per-lane DMA source offsets (bytes from the k0 column of the tile). x
@@ -577,9 +583,29 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
       lds_dma16(wo[u - XL], uniform_ptr(a.wq + (kb + t) * BK),
                 sbase + stage * SB + XB + wave * 1024 + (u - XL) * 8192);
   };
+  // The short last step (K % 16 == 0): chunks past K are not loaded; x gets
+  // zeros there instead, so whatever codes lie in the weight stage (any byte is
+  // a finite code) add nothing. A wave may then issue fewer DMA instructions
+  // than XL + WL, so the waits after it count down to 0.
+  auto issue_short = [&](int t, int stage, int u) {
+    const int k0 = (kb + t) * BK;
+    if (u < XL) {
+      const int row = (u * 8 + wave) * 8 + (lane >> 3);
+      if (k0 + ((lane & 7) ^ ((row >> 1) & 7)) * 8 < a.K) issue_one(t, stage, u);
+      else
+        *reinterpret_cast<u32x4*>(smem + stage * SB + wave * 1024 + u * 8192 + lane * 16) =
+            u32x4{0u, 0u, 0u, 0u};
+    } else {
+      const int row = ((u - XL) * 8 + wave) * 16 + (lane >> 2);
+      if (k0 + ((lane & 3) ^ ((row >> 2) & 3)) * 16 < a.K) issue_one(t, stage, u);
+    }
+  };
   auto issue = [&](int t, int stage) {
 #pragma unroll
-    for (int u = 0; u < XL + WL; ++u) issue_one(t, stage, u);
+    for (int u = 0; u < XL + WL; ++u) {
+      if (!SHORT || t < nkf) issue_one(t, stage, u);
+      else issue_short(t, stage, u);
+    }
   };
 
   // Fragment read offsets within a stage: row r32 of each 32-row tile, lane
@@ -696,7 +722,10 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
     half(fr[1], &fr[0], TN & 1, [&](int i, int p) {
       const int r = i * 2 * TM + p;
       if constexpr (decltype(dma)::value) {
-        if (r < XL + WL) issue_one(t + NS, stage_cur, r);
+        if (r < XL + WL) {
+          if (!SHORT || SC >= 0 || t + NS < nkf) issue_one(t + NS, stage_cur, r);
+          else issue_short(t + NS, stage_cur, r);
+        }
       }
       if (r < 2 * TM + TN) read_one(stage_next, 0, fr[0], r);
       if (r == 2 * TM * TN - 1)
@@ -719,8 +748,8 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
     s_bias[tid] = n < a.N ? bv : 0.0f;
   }
   if (nk > 0) {
-    if (nk > 2) dma_wait_barrier<2 * (XL + WL)>();
-    else if (nk > 1) dma_wait_barrier<XL + WL>();
+    if (nkf > 2) dma_wait_barrier<2 * (XL + WL)>();
+    else if (nkf > 1 && (!SHORT || nk == nkf)) dma_wait_barrier<XL + WL>();
     else dma_wait_barrier<0>();
     read_half(0, 0, fr[0]);
 #pragma unroll
@@ -732,13 +761,13 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
     using SR = std::integral_constant<int, -1>;
     static_assert(NS == 3, "the main loop is unrolled by the stage count");
     // Tile t + 2 in flight, DMA of t + 3.
-    for (; t + NS + 2 < nk; t += NS) {
+    for (; t + NS + 2 < nkf; t += NS) {
       step(t, yes{}, 1, S0{});
       step(t + 1, yes{}, 1, S1{});
       step(t + 2, yes{}, 1, S2{});
     }
     for (; t + NS < nk; ++t) step(t, yes{}, 1, SR{});
-    for (; t + 1 < nk; ++t) step(t, no{}, nk - 2 - t, SR{});
+    for (; t + 1 < nk; ++t) step(t, no{}, !SHORT || nk == nkf ? nk - 2 - t : 0, SR{});
     half(fr[0], &fr[1], 0, [&](int i, int p) {
       const int r = i * 2 * TM + p;
       if (r < 2 * TM + TN) read_one((nk - 1) % NS, 1, fr[1], r);
@@ -851,7 +880,8 @@ void launch_gemm_dma(GemmArgs a, hipStream_t s) {
   a.tiles_m = static_cast<int>(cdiv(a.M, 64 * TM));
   a.tiles_n = static_cast<int>(cdiv(a.N, 256));
   const unsigned grid = static_cast<unsigned>(a.tiles_m) * a.tiles_n;
-  k_gemm_dma<ACT, false, TM><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
+  if (a.K % 64) k_gemm_dma<ACT, false, TM, kDmaTN, 2, true><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
+  else k_gemm_dma<ACT, false, TM><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
 }
 
 // 128 x 128 tiles, whole (k_gemm_dma128): 98 VGPRs and 74 KiB of LDS, so two
@@ -861,7 +891,8 @@ void launch_gemm_dma128(GemmArgs a, hipStream_t s) {
   a.tiles_m = static_cast<int>(cdiv(a.M, 128));
   a.tiles_n = static_cast<int>(cdiv(a.N, 128));
   const unsigned grid = static_cast<unsigned>(a.tiles_m) * a.tiles_n;
-  k_gemm_dma<ACT, false, 2, 1, 2><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
+  if (a.K % 64) k_gemm_dma<ACT, false, 2, 1, 2, true><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
+  else k_gemm_dma<ACT, false, 2, 1, 2><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
 }
 
 // Split-K finish: each thread takes two partial f4 of a tail tile, kBlock
@@ -1055,12 +1086,13 @@ void launch_gemm_dma_splitk(GemmArgs a, const DmaPlan& p, hipStream_t s) {
   a.tiles_m = static_cast<int>(cdiv(a.M, 64 * TM));
   a.tiles_n = static_cast<int>(cdiv(a.N, 256));
   a.full_tiles = p.full;
-  const int nk = a.K / 64;
+  const int nk = static_cast<int>(cdiv(a.K, 64LL));
   a.split_steps = static_cast<int>(cdiv(nk, p.splits));
   a.splits = static_cast<int>(cdiv(nk, a.split_steps));   // no empty ranges
   const int rest = a.tiles_m * a.tiles_n - a.full_tiles;
   const unsigned grid = static_cast<unsigned>(a.full_tiles + rest * a.splits);
-  k_gemm_dma<ACT, true, TM><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
+  if (a.K % 64) k_gemm_dma<ACT, true, TM, kDmaTN, 2, true><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
+  else k_gemm_dma<ACT, true, TM><<<dim3(grid), dim3(kDmaThreads), 0, s>>>(a);
   const int64_t n4 = static_cast<int64_t>(rest) * 8 * kDmaTN * TM * 4 * 64;
   const dim3 rgrid(static_cast<unsigned>(cdiv(n4, kBlock * kReduceF4)));
   if (a.n_out > 0) k_splitk_reduce<ACT, TM, true><<<rgrid, dim3(kBlock), 0, s>>>(a);
@@ -1674,7 +1706,7 @@ __global__ __launch_bounds__(kBlock) void k_general_reduce(GenArgs a) {
 //   M <= 64       k_stream<2 or 4> under the same size rules (3 row tiles
 //                 per workgroup); else k_skinny, TM = ceil(M / 16); for
 //                 M > 24 and K > 8192 the split k_gemm_dma plan below first
-//   M > 64        k_gemm_dma (K % 64 == 0 and 32-bit operand offsets) with
+//   M > 64        k_gemm_dma (32-bit operand offsets) with
 //                 the x tile (256 or 128 rows) and split-K plan of dma_plan:
 //                 the last, short wave of tiles split over K (2-16 k-ranges,
 //                 partial tiles in the workspace, k_splitk_reduce) when the
@@ -1683,7 +1715,7 @@ __global__ __launch_bounds__(kBlock) void k_general_reduce(GenArgs a) {
 //                 (k_gemm_dma128, no partials) is modelled faster;
 //   M > 64        else k_gemm_dma without a split (x tile of dma_plan), or
 //                 k_gemm_dma128 where modelled faster; without k_gemm_dma
-//                 (K % 64 != 0 or offsets past 32 bits) k_gemm 128 x 64 x 64,
+//                 (offsets past 32 bits) k_gemm 128 x 64 x 64,
 //                 2 x 2 waves (M >= 1024: 256 x 256 x 64, 4 x 2 waves)
 enum Kind { kSkinny1, kSkinny2, kSkinny4, kTileMid, kTileLarge, kTileDma, kStream1, kStream2,
             kStream4, kTileDmaSplit, kTileDma128 };
@@ -1695,10 +1727,12 @@ bool stream_ok(int64_t M, int64_t N, int64_t K) {
 }
 
 // k_gemm_dma addresses x and wq with 32-bit byte offsets from a scalar base
-// and needs whole 64-k steps.
+// and 16-byte rows. K % 64 != 0 ends in a short step: bf16 M = 334, N = 12288,
+// K = 3312 104.0 -> 42.7 us, M = 2753, N = 421, K = 3440 180.5 -> 28.6, M = 65,
+// N = 256, K = 272 12.0 -> 8.9 (k_gemm before).
 bool dma_ok(int64_t M, int64_t N, int64_t K) {
   constexpr int64_t kLim = (1LL << 32) - 4096;
-  return K % 64 == 0 && M * K * 2 < kLim && N * K < kLim;
+  return K % 16 == 0 && M * K * 2 < kLim && N * K < kLim;
 }
 
 // Plan of the k_gemm_dma path with the lowest modelled time (0.01 us): the
@@ -1724,7 +1758,7 @@ int64_t dma_step_cost(int tm, int64_t wgs, int64_t cus) {
 }
 
 DmaPlan dma_plan(int64_t M, int64_t N, int64_t K, bool allow_split, int64_t* cost = nullptr) {
-  const int64_t cus = device_cus(), nk = K / 64;
+  const int64_t cus = device_cus(), nk = cdiv(K, 64LL);
   DmaPlan best{4, 0, 1};
   int64_t best_cost = INT64_MAX;
   for (const int tm : {4, 2, 3}) {
@@ -1770,7 +1804,7 @@ DmaPlan dma_plan(int64_t M, int64_t N, int64_t K, bool allow_split, int64_t* cos
 // 138.0; M = 200, N = 50000, K = 2048: 53.4 against 64.5).
 int64_t dma128_cost(int64_t M, int64_t N, int64_t K) {
   const int64_t cus = device_cus();
-  const int64_t tiles = cdiv(M, 128) * cdiv(N, 128), nk = K / 64;
+  const int64_t tiles = cdiv(M, 128) * cdiv(N, 128), nk = cdiv(K, 64LL);
   if (M <= 64) return INT64_MAX;
   if (tiles <= cus) return 780 + nk * (46 + 19 * tiles / cus);
   return 780 + nk * 120 * cdiv(tiles, 2 * cus);
