@@ -45,7 +45,7 @@
 // accumulators. Split tiles leave them to k_splitk_reduce, which stages the
 // same operands per workgroup and adds them per output.
 //
-// k_stream1<ACT> (M <= 16) and k_stream<ACT, TM> (M <= 64): persistent
+// k_decode (M <= 32), k_stream1 (M <= 16) and k_stream<ACT, TM> (M <= 64):
 // weight streaming for large weights (see the kernels' comments).
 //
 // k_skinny<ACT, TM, TN, U> (M <= 64): weight streaming with the K split across
@@ -1381,10 +1381,9 @@ __global__ __launch_bounds__(64 * kStreamWaves) void k_stream(GemmArgs a) {
   }
 }
 
-// k_stream1<ACT, RT> (M <= 16): weight streaming with row-contiguous loads.
+// k_stream1<ACT> (M <= 16): weight streaming with row-contiguous loads.
 //
-// One 16-wave workgroup owns RT consecutive row tiles (16 RT weight rows;
-// RT = 3, or 4 when 48-row workgroups would outnumber the CUs). Every wave
+// One 16-wave workgroup owns RT = 3 consecutive row tiles (48 weight rows). Every wave
 // issues all of its weight loads at once, as 1 KiB row-contiguous requests
 // (wave w: rows RT w .. RT w + RT - 1, step by step; 64 lanes x 16 bytes per
 // request), which stream from HBM far faster than MFMA-shaped requests
@@ -1398,12 +1397,12 @@ __global__ __launch_bounds__(64 * kStreamWaves) void k_stream(GemmArgs a) {
 // M <= 16.
 constexpr int kStream1Stride = 1040;
 constexpr int kStream1MaxSteps = 4;
-constexpr int kStream1MaxRT = 4;   // two stages of 64 rows: 130 KiB of LDS
+constexpr int kStream1RT = 3;
 
-template <int ACT, int RT>
+template <int ACT>
 __global__ __launch_bounds__(1024) void k_stream1(GemmArgs a) {
+  constexpr int RT = kStream1RT;
   constexpr int ROWS = 16 * RT, SB = ROWS * kStream1Stride, NST = kStream1MaxSteps;
-  static_assert(RT >= 3 && RT <= kStream1MaxRT, "3 or 4 row tiles");
   static_assert(2 * SB <= 160 * 1024, "two LDS stages");
   static_assert(16 * RT * 64 * 16 <= 2 * SB, "reduction fits in the stages");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * SB];
@@ -1511,24 +1510,211 @@ __global__ __launch_bounds__(1024) void k_stream1(GemmArgs a) {
   }
 }
 
-// Row tiles per k_stream1 workgroup: 3 while 48-row workgroups fit on the
-// CUs at once, else 4 (0: neither fits; the host picks another kernel).
-// Measured on MI355X, M = 16, K = 4096, N = 14336: 299 workgroups of 48 rows
-// do not fit, and the kernel it then fell back to (k_skinny) took 30.0 us;
-// 224 workgroups of 64 rows took 23.8 us.
-int stream1_tiles(int64_t N) {
+// k_decode<ACT, RT, MT, NBC> (M <= 32): weight streaming for any K % 16 == 0.
+//
+// An 8-wave workgroup owns RT row tiles (16 RT weight rows); wave w takes the
+// 128-k blocks w, w + 8, ... of all of them. A (block, row tile) unit is two
+// loads of 8 rows x 128 bytes per wave straight from HBM (as fast as 1 KiB
+// row-contiguous requests; the MFMA operand's own 16 rows x 64 bytes stream 20%
+// slower), D RT units in flight per wave (96 KiB or more per CU). A unit goes
+// through a 2 KiB stage of the wave's own in LDS into the MFMA layout (16-byte
+// chunk c of row r at c ^ (r & 7): no bank conflicts; LDS operations of a wave
+// are in order, so no barrier) and is widened and multiplied. x is staged by
+// LDS DMA in chunks of KC = 1024 NBC columns (NBC blocks per wave; 16-byte chunk
+// c of row m at c ^ (m & 7)), double buffered: one barrier per chunk, then the
+// next chunk's DMA, waited for by count, so that the weight loads stay in
+// flight. The waves' partial tiles are summed in wave order (deterministic)
+// through LDS.
+//
+// Bound: the weight stream. Timing-only copies at N = 4096, K = 11008, M = 1:
+// loads alone 13.4 us of 15.1, without the transpose through LDS 14.2, without
+// the multiplications 13.8 (k_skinny, which this replaces there: 19.6). 16 waves
+// with half the units each: 13.9-15.2 against 14.9-15.9 us there, slower on
+// other shapes. x costs throughput, not latency (M = 16: 22.4 us, every
+// workgroup stages all of x): four 32 KiB buffers instead of two of 64, 23.9.
+//
+// Columns past K: x is zero there in LDS, the weight loads are clamped (any
+// byte is a finite code); rows past M repeat row M - 1, rows past N row N - 1,
+// and are not stored.
+constexpr int kDecWaves = 8;
+constexpr int kDecXBytes = 64 * 1024;      // one x buffer
+constexpr int decode_depth(int rt) { return rt == 1 ? 8 : rt == 2 ? 4 : rt == 3 ? 3 : rt <= 6 ? 2 : 1; }
+
+template <int ACT, int RT, int MT, int NBC>
+__global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
+  constexpr int KC = 1024 * NBC, RS = KC * 2;        // columns, row bytes
+  constexpr int MP = kDecXBytes / RS;                // rows of an x chunk
+  constexpr int D = decode_depth(RT);                // blocks in flight per wave
+  static_assert(MP <= 16 * MT, "x rows");
+  __shared__ __attribute__((aligned(1024))) uint8_t sx[2 * kDecXBytes];
+  __shared__ __attribute__((aligned(1024))) uint8_t sw[kDecWaves * 2048];
+  static_assert(kDecWaves * RT * MT * 1024 <= 2 * kDecXBytes, "partial tiles fit in the x buffers");
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * RT;
+  const uint32_t sbase = __builtin_amdgcn_readfirstlane(lds_addr(sx));
+  uint8_t* const st = sw + wave * 2048;
+  const int nblk = (a.K + 127) / 128, nchunk = (a.K + KC - 1) / KC;
+  const int iters = (nblk + kDecWaves - 1) / kDecWaves;   // blocks per wave, the same for all
+
+  // Chunk c of x: 1 KiB of one row per wave instruction.
+  auto stage_x = [&](int c) {
+    const int c0 = c * KC, len = min(KC, a.K - c0);
+    const int segs = (len + 511) / 512, total = a.M * segs;
+    for (int q = wave; q < total; q += kDecWaves) {
+      const int m = q / segs, sg = q - m * segs;
+      const int col = sg * 512 + ((lane ^ (m & 7)) * 8);       // source column of the lane's slot
+      const uint32_t dst = (c & 1) * kDecXBytes + m * RS + sg * 1024;
+      if (col < len)
+        lds_dma16(static_cast<uint32_t>(col) * 2u,
+                  uniform_ptr(a.x + static_cast<int64_t>(m) * a.K + c0), sbase + dst);
+      else
+        *reinterpret_cast<u32x4*>(sx + dst + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  // Unit loads: rows 8 h + lane / 8 of tile r, 16 bytes at chunk lane % 8.
+  const int8_t* wrow[RT][2];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      wrow[r][h] = a.wq + static_cast<int64_t>(min(n0 + r * 16 + h * 8 + (lane >> 3), a.N - 1)) * a.K;
+  u32x4 w[D][RT][2];
+  auto load = [&](int i, int d, int r) {
+    const int k = min((i * kDecWaves + wave) * 128 + (lane & 7) * 16, a.K - 16);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      w[d][r][h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow[r][h] + k));
+  };
+
+  f4 acc[RT][MT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[r][j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  stage_x(0);
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+#pragma unroll
+    for (int r = 0; r < RT; ++r) load(d, d, r);
+
+  // Before a chunk: at most the weight loads issued after its DMA outstanding.
+  constexpr int kFirst = 2 * D * RT < 63 ? 2 * D * RT : 63;
+  constexpr int kLater = 2 * NBC * RT < 63 ? 2 * NBC * RT : 63;
+  const int wpos = (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);   // + 1024 for h = 1
+  uint32_t xa[MT];                                    // x row of the lane (rows past M repeat)
+#pragma unroll
+  for (int j = 0; j < MT; ++j) xa[j] = min(j * 16 + row, a.M - 1);
+  u32x4 fw[2], xf[MT][4];
+  auto multiply = [&](int r) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      uint32_t o[8];
+      i8x4_to_act<ACT>(fw[e].x, o[0], o[1]);
+      i8x4_to_act<ACT>(fw[e].y, o[2], o[3]);
+      i8x4_to_act<ACT>(fw[e].z, o[4], o[5]);
+      i8x4_to_act<ACT>(fw[e].w, o[6], o[7]);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        acc[r][j] = mfma16x16x32<ACT>(u32x4{o[0], o[1], o[2], o[3]}, xf[j][2 * e], acc[r][j]);
+        acc[r][j] = mfma16x16x32<ACT>(u32x4{o[4], o[5], o[6], o[7]}, xf[j][2 * e + 1], acc[r][j]);
+      }
+    }
+  };
+  for (int i0 = 0; i0 < iters; i0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int i = i0 + d;
+      if (i < iters) {
+        const int c = i / NBC;
+        if (i % NBC == 0) {
+          if (i == 0) dma_wait_barrier<kFirst>();
+          else dma_wait_barrier<kLater>();
+          if (c + 1 < nchunk) stage_x(c + 1);
+        }
+        const int b = i * kDecWaves + wave;
+        const uint8_t* xb = sx + (c & 1) * kDecXBytes;
+        const int kc = (b * 128 - c * KC) >> 3;         // first 8-value chunk of the block
+        const bool live = b < nblk;
+        if (live) {
+#pragma unroll
+          for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int ch = kc + ((e >> 1) * 4 + g) * 2 + (e & 1);
+              xf[j][e] = *reinterpret_cast<const u32x4*>(xb + xa[j] * RS + ((ch ^ (xa[j] & 7)) << 4));
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          *reinterpret_cast<u32x4*>(st + wpos) = w[d][r][0];
+          *reinterpret_cast<u32x4*>(st + 1024 + wpos) = w[d][r][1];
+          fw[0] = *reinterpret_cast<const u32x4*>(st + row * 128 + ((g ^ (row & 7)) << 4));
+          fw[1] = *reinterpret_cast<const u32x4*>(st + row * 128 + (((g + 4) ^ (row & 7)) << 4));
+          load(i + D, d, r);
+          if (live) multiply(r);
+        }
+      }
+    }
+  }
+
+  // Partial tiles through LDS; wave p sums pairs p, p + 8, ... of (tile, m-tile).
+  dma_wait_barrier<0>();
+  f4* red = reinterpret_cast<f4*>(sx);
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) red[((r * MT + j) * kDecWaves + wave) * 64 + lane] = acc[r][j];
+  __syncthreads();
+  const bool vec_store = (a.N % 4) == 0;
+  for (int p = wave; p < RT * MT; p += kDecWaves) {
+    const int r = p / MT, m = (p % MT) * 16 + row, nq = n0 + r * 16 + g * 4;
+    if (m >= a.M || nq >= a.N) continue;
+    const f4* src = red + p * kDecWaves * 64 + lane;
+    f4 sum = src[0];
+#pragma unroll
+    for (int v = 1; v < kDecWaves; ++v) sum += src[v * 64];
+    store_quad<ACT>(a, sum, m, nq, vec_store);
+  }
+}
+
+// Row tiles per k_decode workgroup: the fewest that leave at most one
+// workgroup per CU (at most 8).
+int decode_tiles(int64_t N) {
   const int64_t cus = device_cus();
-  if (cdiv(N, 48) <= cus) return 3;
-  if (cdiv(N, 16 * kStream1MaxRT) <= cus) return kStream1MaxRT;
-  return 0;
+  for (const int rt : {1, 2, 3, 4, 6})
+    if (cdiv(N, 16 * rt) <= cus) return rt;
+  return 8;
+}
+
+template <int ACT, int RT>
+void launch_decode_rt(const GemmArgs& a, hipStream_t s) {
+  const dim3 g(static_cast<unsigned>(cdiv(a.N, 16 * RT))), b(64 * kDecWaves);
+  if (a.M <= 4) k_decode<ACT, RT, 1, 8><<<g, b, 0, s>>>(a);
+  else if (a.M <= 8) k_decode<ACT, RT, 1, 4><<<g, b, 0, s>>>(a);
+  else if (a.M <= 16) k_decode<ACT, RT, 1, 2><<<g, b, 0, s>>>(a);
+  else k_decode<ACT, RT, 2, 1><<<g, b, 0, s>>>(a);
 }
 
 template <int ACT>
-void launch_stream1(GemmArgs a, hipStream_t s) {
-  const int rt = stream1_tiles(a.N);
-  const unsigned grid = static_cast<unsigned>(cdiv(a.N, 16 * rt));
-  if (rt == 3) k_stream1<ACT, 3><<<dim3(grid), dim3(1024), 0, s>>>(a);
-  else k_stream1<ACT, kStream1MaxRT><<<dim3(grid), dim3(1024), 0, s>>>(a);
+void launch_decode(const GemmArgs& a, hipStream_t s) {
+  switch (decode_tiles(a.N)) {
+    case 1: launch_decode_rt<ACT, 1>(a, s); break;
+    case 2: launch_decode_rt<ACT, 2>(a, s); break;
+    case 3: launch_decode_rt<ACT, 3>(a, s); break;
+    case 4: launch_decode_rt<ACT, 4>(a, s); break;
+    case 6: launch_decode_rt<ACT, 6>(a, s); break;
+    default: launch_decode_rt<ACT, 8>(a, s); break;
+  }
+}
+
+template <int ACT>
+void launch_stream1(const GemmArgs& a, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(cdiv(a.N, 16 * kStream1RT));
+  k_stream1<ACT><<<dim3(grid), dim3(1024), 0, s>>>(a);
 }
 
 template <int ACT, int TM>
@@ -1700,9 +1886,10 @@ __global__ __launch_bounds__(kBlock) void k_general_reduce(GenArgs a) {
 // Host side
 // ---------------------------------------------------------------------------
 // Kernel choice by M (measured on MI355X at N = 11008, K = 4096):
+//   M <= 32       k_decode for weights of at least 8 MB (see decode_ok), else:
 //   M <= 16       k_stream1 when the weight is at least 8 MB, K % 1024 == 0,
-//                 K <= 4096 and the 48-row (else 64-row) groups fit one
-//                 wave of workgroups; else k_skinny (TM = 1)
+//                 K <= 4096 and 48-row groups just fit one wave of workgroups;
+//                 else k_skinny (TM = 1)
 //   M <= 64       k_stream<2 or 4> under the same size rules (3 row tiles
 //                 per workgroup); else k_skinny, TM = ceil(M / 16); for
 //                 M > 24 and K > 8192 the split k_gemm_dma plan below first
@@ -1718,12 +1905,34 @@ __global__ __launch_bounds__(kBlock) void k_general_reduce(GenArgs a) {
 //                 (offsets past 32 bits) k_gemm 128 x 64 x 64,
 //                 2 x 2 waves (M >= 1024: 256 x 256 x 64, 4 x 2 waves)
 enum Kind { kSkinny1, kSkinny2, kSkinny4, kTileMid, kTileLarge, kTileDma, kStream1, kStream2,
-            kStream4, kTileDmaSplit, kTileDma128 };
+            kStream4, kTileDmaSplit, kTileDma128, kDecode };
 
 // The streaming kernels pay a fixed cost for their large workgroups; below
 // 8 MB of weight the k_skinny kernels are faster.
 bool stream_ok(int64_t M, int64_t N, int64_t K) {
   return K % 1024 == 0 && N * K >= (8LL << 20) && M * K * 2 < (1LL << 31);
+}
+
+// Whether k_decode takes M <= 32 (24 < M with K > 8192 goes to the split tiles
+// first). Below 8 MB of weight k_skinny is level or faster (N = 512, K = 768: 3.7
+// against 4.5 us; 2176, 2560: 7.0 each). With three row tiles per workgroup
+// k_stream1 / k_stream<2> stay ahead where they apply (N = 11008, K = 4096, M =
+// 16: 14.2 against 15.2 us; M = 32: 18.6 against 18.9); with one row tile and a
+// long K every workgroup stages more x than weight (N = 4096, K = 11008, M = 16:
+// k_skinny 21.2 against 22.4; M = 8: 20.6 against 17.9). Elsewhere (fp16, us):
+// M = 4, N = 4096, K = 11008 20.4 -> 16.0; N = K = 4096 10.7 -> 8.5; N = 14336
+// 18.7 -> 16.3; N = 8832, K = 5440 24.4 -> 17.2; N = 32000, M = 16 52.7 -> 30.2;
+// N = 5120, K = 13824 43.3 -> 27.9; M = 24, N = 14336 35.0 -> 19.7.
+bool decode_ok(int64_t M, int64_t N, int64_t K) {
+  if (M > 32 || N * K < (8LL << 20) || M * K * 2 >= (1LL << 31)) return false;
+  const int rt = decode_tiles(N);
+  if (stream_ok(M, N, K)) {
+    if (rt == 3 && (M > 16 || K <= 4096)) return false;
+    // k_stream<2>: M = 32, N = 5000, K = 2048 9.1 against 9.8 us (M = 24, N = 8192,
+    // K = 4096 16.8 against 15.7)
+    if (rt == 2 && M > 16 && (M > 24 || K < 4096)) return false;
+  }
+  return !(rt == 1 && M > 8 && K > 8192);
 }
 
 // k_gemm_dma addresses x and wq with 32-bit byte offsets from a scalar base
@@ -1833,12 +2042,13 @@ DmaPlan split_plan(int64_t M, int64_t N, int64_t K) {
 Kind choose(int64_t M, int64_t N, int64_t K, int64_t n_out, size_t ws_bytes, DmaPlan& plan) {
   const int64_t cus = device_cus();
   const bool stream = stream_ok(M, N, K);
+  const bool decode = decode_ok(M, N, K);
   if (M <= 16)
-    return (stream && K <= 4096 && stream1_tiles(N) > 0) ? kStream1 : kSkinny1;
+    return decode ? kDecode : (stream && K <= 4096 && decode_tiles(N) == 3) ? kStream1 : kSkinny1;
   const bool tiles_fit = cdiv(N, 16) <= kStreamMaxTiles * cus;
   const Kind narrow = M <= 32 ? ((stream && tiles_fit) ? kStream2 : kSkinny2)
                               : ((stream && tiles_fit) ? kStream4 : kSkinny4);
-  if (M <= 64 && !dma_candidate(M, N, K)) return narrow;
+  if (M <= 64 && !dma_candidate(M, N, K)) return decode ? kDecode : narrow;
   if (!dma_ok(M, N, K)) return M < 1024 ? kTileMid : kTileLarge;
   int64_t cost = 0;
   plan = dma_plan(M, N, K, true, &cost);
@@ -1869,6 +2079,7 @@ void launch_kind(Kind k, const GemmArgs& a, const DmaPlan& p, hipStream_t s) {
     case kSkinny1: launch_skinny<ACT, 1, 1, 4>(a, s); break;
     case kSkinny2: launch_skinny<ACT, 2, 1, 4>(a, s); break;
     case kSkinny4: launch_skinny<ACT, 4, 1, 2>(a, s); break;
+    case kDecode: launch_decode<ACT>(a, s); break;
     case kStream1: launch_stream1<ACT>(a, s); break;
     case kStream2: launch_stream<ACT, 2>(a, s); break;
     case kStream4: launch_stream<ACT, 4>(a, s); break;
