@@ -137,6 +137,8 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   int splits, split_steps;  // split-K: number of k-ranges, 64-k steps per range
   int full_tiles;           // split-K: tiles [0, full_tiles) run whole, the rest split
+  const uint16_t* xp;       // k_decode: x as [M, ldx], 16-byte rows (x itself, or padded with zeros)
+  int ldx;
 };
 
 // Workgroup b of n goes to XCD b % 8; renumbered so that each XCD takes a
@@ -1510,7 +1512,7 @@ __global__ __launch_bounds__(1024) void k_stream1(GemmArgs a) {
   }
 }
 
-// k_decode<ACT, RT, MT, NBC> (M <= 32): weight streaming for any K % 16 == 0.
+// k_decode<ACT, RT, MT, NBC> (M <= 32): weight streaming for any K >= 16.
 //
 // An 8-wave workgroup owns RT row tiles (16 RT weight rows); wave w takes the
 // 128-k blocks w, w + 8, ... of all of them. A (block, row tile) unit is two
@@ -1538,9 +1540,10 @@ __global__ __launch_bounds__(1024) void k_stream1(GemmArgs a) {
 // and are not stored.
 constexpr int kDecWaves = 8;
 constexpr int kDecXBytes = 64 * 1024;      // one x buffer
+typedef u32x4 __attribute__((aligned(1))) u32x4_any;
 constexpr int decode_depth(int rt) { return rt == 1 ? 8 : rt == 2 ? 4 : rt == 3 ? 3 : rt <= 6 ? 2 : 1; }
 
-template <int ACT, int RT, int MT, int NBC>
+template <int ACT, int RT, int MT, int NBC, bool ANY>   // ANY: K % 16 != 0
 __global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
   constexpr int KC = 1024 * NBC, RS = KC * 2;        // columns, row bytes
   constexpr int MP = kDecXBytes / RS;                // rows of an x chunk
@@ -1561,7 +1564,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
 
   // Chunk c of x: 1 KiB of one row per wave instruction.
   auto stage_x = [&](int c) {
-    const int c0 = c * KC, len = min(KC, a.K - c0);
+    const int c0 = c * KC, len = min(KC, a.ldx - c0);
     const int segs = (len + 511) / 512, total = a.M * segs;
     for (int q = wave; q < total; q += kDecWaves) {
       const int m = q / segs, sg = q - m * segs;
@@ -1569,12 +1572,15 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
       const uint32_t dst = (c & 1) * kDecXBytes + m * RS + sg * 1024;
       if (col < len)
         lds_dma16(static_cast<uint32_t>(col) * 2u,
-                  uniform_ptr(a.x + static_cast<int64_t>(m) * a.K + c0), sbase + dst);
+                  uniform_ptr(a.xp + static_cast<int64_t>(m) * a.ldx + c0), sbase + dst);
       else
         *reinterpret_cast<u32x4*>(sx + dst + lane * 16) = u32x4{0u, 0u, 0u, 0u};
     }
   };
-  // Unit loads: rows 8 h + lane / 8 of tile r, 16 bytes at chunk lane % 8.
+  // Unit loads: rows 8 h + lane / 8 of tile r, 16 bytes at chunk lane % 8. ANY:
+  // rows without alignment; a load past K reads on into the next row, and the
+  // last row's loads end with the weight. (Instances of their own: the checks
+  // cost the others 6-18%.)
   const int8_t* wrow[RT][2];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
@@ -1583,10 +1589,32 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
       wrow[r][h] = a.wq + static_cast<int64_t>(min(n0 + r * 16 + h * 8 + (lane >> 3), a.N - 1)) * a.K;
   u32x4 w[D][RT][2];
   auto load = [&](int i, int d, int r) {
-    const int k = min((i * kDecWaves + wave) * 128 + (lane & 7) * 16, a.K - 16);
+    const int k = (i * kDecWaves + wave) * 128 + (lane & 7) * 16;
 #pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if constexpr (ANY) {
+        const bool last = n0 + r * 16 + h * 8 + (lane >> 3) >= a.N - 1;
+        w[d][r][h] = __builtin_nontemporal_load(
+            reinterpret_cast<const u32x4_any*>(wrow[r][h] + min(k, last ? a.K - 16 : a.K - 1)));
+      } else {
+        w[d][r][h] = __builtin_nontemporal_load(
+            reinterpret_cast<const u32x4*>(wrow[r][h] + min(k, a.K - 16)));
+      }
+    }
+  };
+  // The last row's partly valid chunk (K % 16 != 0) was loaded from 16 bytes
+  // before its end: moved down to where the chunk starts (its end is never read
+  // against a non-zero x).
+  auto place_last = [&](int r, const u32x4 (&v)[2], uint8_t* stage, int wp) {
+    const int k = a.K / 128 * 128 + (lane & 7) * 16;
+    if (k >= a.K || k + 16 <= a.K) return;
     for (int h = 0; h < 2; ++h)
-      w[d][r][h] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow[r][h] + k));
+      if (n0 + r * 16 + h * 8 + (lane >> 3) >= a.N - 1) {
+        const uint32_t words[4] = {v[h].x, v[h].y, v[h].z, v[h].w};
+        for (int j = k + 16 - a.K; j < 16; ++j)
+          stage[h * 1024 + wp + j - (k + 16 - a.K)] =
+              static_cast<uint8_t>(words[j >> 2] >> (8 * (j & 3)));
+      }
   };
 
   f4 acc[RT][MT];
@@ -1652,6 +1680,9 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
         for (int r = 0; r < RT; ++r) {
           *reinterpret_cast<u32x4*>(st + wpos) = w[d][r][0];
           *reinterpret_cast<u32x4*>(st + 1024 + wpos) = w[d][r][1];
+          if constexpr (ANY) {
+            if (b == nblk - 1) place_last(r, w[d][r], st, wpos);
+          }
           fw[0] = *reinterpret_cast<const u32x4*>(st + row * 128 + ((g ^ (row & 7)) << 4));
           fw[1] = *reinterpret_cast<const u32x4*>(st + row * 128 + (((g + 4) ^ (row & 7)) << 4));
           load(i + D, d, r);
@@ -1690,24 +1721,32 @@ int decode_tiles(int64_t N) {
   return 8;
 }
 
-template <int ACT, int RT>
+template <int ACT, int RT, bool ANY>
 void launch_decode_rt(const GemmArgs& a, hipStream_t s) {
   const dim3 g(static_cast<unsigned>(cdiv(a.N, 16 * RT))), b(64 * kDecWaves);
-  if (a.M <= 4) k_decode<ACT, RT, 1, 8><<<g, b, 0, s>>>(a);
-  else if (a.M <= 8) k_decode<ACT, RT, 1, 4><<<g, b, 0, s>>>(a);
-  else if (a.M <= 16) k_decode<ACT, RT, 1, 2><<<g, b, 0, s>>>(a);
-  else k_decode<ACT, RT, 2, 1><<<g, b, 0, s>>>(a);
+  if (a.M <= 4) k_decode<ACT, RT, 1, 8, ANY><<<g, b, 0, s>>>(a);
+  else if (a.M <= 8) k_decode<ACT, RT, 1, 4, ANY><<<g, b, 0, s>>>(a);
+  else if (a.M <= 16) k_decode<ACT, RT, 1, 2, ANY><<<g, b, 0, s>>>(a);
+  else k_decode<ACT, RT, 2, 1, ANY><<<g, b, 0, s>>>(a);
 }
 
 template <int ACT>
 void launch_decode(const GemmArgs& a, hipStream_t s) {
-  switch (decode_tiles(a.N)) {
-    case 1: launch_decode_rt<ACT, 1>(a, s); break;
-    case 2: launch_decode_rt<ACT, 2>(a, s); break;
-    case 3: launch_decode_rt<ACT, 3>(a, s); break;
-    case 4: launch_decode_rt<ACT, 4>(a, s); break;
-    case 6: launch_decode_rt<ACT, 6>(a, s); break;
-    default: launch_decode_rt<ACT, 8>(a, s); break;
+  const int rt = decode_tiles(a.N);
+  if (a.K % 16) {   // fewer instances
+    if (rt == 1) launch_decode_rt<ACT, 1, true>(a, s);
+    else if (rt == 2) launch_decode_rt<ACT, 2, true>(a, s);
+    else if (rt <= 4) launch_decode_rt<ACT, 4, true>(a, s);
+    else launch_decode_rt<ACT, 8, true>(a, s);
+    return;
+  }
+  switch (rt) {
+    case 1: launch_decode_rt<ACT, 1, false>(a, s); break;
+    case 2: launch_decode_rt<ACT, 2, false>(a, s); break;
+    case 3: launch_decode_rt<ACT, 3, false>(a, s); break;
+    case 4: launch_decode_rt<ACT, 4, false>(a, s); break;
+    case 6: launch_decode_rt<ACT, 6, false>(a, s); break;
+    default: launch_decode_rt<ACT, 8, false>(a, s); break;
   }
 }
 
@@ -1723,6 +1762,42 @@ void launch_stream(GemmArgs a, hipStream_t s) {
   int grid = std::min(tiles, device_cus());
   grid = std::max(grid, static_cast<int>(cdiv(tiles, kStreamMaxTiles)));
   k_stream<ACT, TM><<<dim3(static_cast<unsigned>(grid)), dim3(64 * kStreamWaves), 0, s>>>(a);
+}
+
+// Rows of kb bytes -> rows of ld bytes (ld % 16 == 0), zero-padded, for two
+// buffers in one launch: any alignment of the source, one 16-byte chunk of the
+// destination per thread and step; a chunk that the source does not hold whole
+// is read by bytes. Bound by memory: [11008, 4090] codes 45 MB read and written.
+struct PadArgs {
+  const uint8_t* src[2];
+  uint8_t* dst[2];
+  int64_t rows[2], kb[2], ld[2];
+};
+__global__ __launch_bounds__(kBlock) void k_pad_rows(PadArgs a) {
+  const int64_t n0 = a.rows[0] * (a.ld[0] >> 4), n = n0 + a.rows[1] * (a.ld[1] >> 4);
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * kBlock) {
+    const int p = i >= n0;
+    const int64_t c = p ? i - n0 : i, cpr = a.ld[p] >> 4, r = c / cpr, k = (c - r * cpr) * 16;
+    const uint8_t* s = a.src[p] + r * a.kb[p] + k;
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (k + 16 <= a.kb[p]) {
+      v = *reinterpret_cast<const u32x4_any*>(s);
+    } else {
+      uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (k + j < a.kb[p]) w[j >> 2] |= static_cast<uint32_t>(s[j]) << (8 * (j & 3));
+      v = u32x4{w[0], w[1], w[2], w[3]};
+    }
+    *reinterpret_cast<u32x4*>(a.dst[p] + r * a.ld[p] + k) = v;
+  }
+}
+
+void launch_pad(const PadArgs& a, hipStream_t s) {
+  const int64_t n = a.rows[0] * (a.ld[0] >> 4) + a.rows[1] * (a.ld[1] >> 4);
+  const int64_t g = std::min<int64_t>(cdiv(n, static_cast<int64_t>(kBlock)), 16LL * device_cus());
+  k_pad_rows<<<dim3(static_cast<unsigned>(g)), dim3(kBlock), 0, s>>>(a);
 }
 
 // Any shape or activation dtype (fp32 activations, K not a multiple of 16,
@@ -2167,10 +2242,87 @@ bool mfma_path(int64_t M, int64_t N, int64_t K, const void* x, const int8_t* wq,
          N < (1LL << 30) && K < (1LL << 30) && cdiv(M, 64) * cdiv(N, 64) < (1LL << 31);
 }
 
+// fp16 / bf16 with K % 16 != 0 on the MFMA kernels: the rows of x zero-padded to
+// a multiple of 16 in the workspace and the weight either read as it is
+// (k_decode, M <= 32 and 8 MB or more) or padded too. Against the fp32 FMA
+// kernel (k_w8a16_general), GPU time of a call: see w8a16_padded.
+bool pad_direct(int64_t M, int64_t N, int64_t K) { return M <= 32 && N * K >= (8LL << 20) && K >= 16; }
+
+int64_t pad_align(int64_t v) { return cdiv(v, 256LL) * 256; }
+
+int64_t pad_bytes(int64_t M, int64_t N, int64_t K) {
+  const int64_t kp = cdiv(K, 16LL) * 16;
+  const int64_t xb = pad_align(M * kp * 2);
+  if (pad_direct(M, N, K)) return xb;
+  return xb + pad_align(N * kp) + splitk_bytes(M, N, split_plan(M, N, kp));
+}
+
+// Whether the 32-bit sizes and offsets of the MFMA kernels hold.
+bool pad_ok(int64_t M, int64_t N, int64_t K) {
+  return K % 16 != 0 && N * K >= 4096 && M < (1LL << 30) && N < (1LL << 30) && K < (1LL << 29) &&
+         cdiv(M, 64) * cdiv(N, 64) < (1LL << 31) && (!pad_direct(M, N, K) || M * (K + 16) * 2 < (1LL << 31));
+}
+
+template <int ACT>
+int w8a16_t(const void* x, const int8_t* wq, const void* scales, const void* bias,
+            const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N, int64_t K,
+            void* ws, size_t ws_bytes, void* y, hipStream_t s);
+
+// bf16, M = 16, N = 9000, K = 5000 131.7 -> 24.7 us; M = 108, N = 7386, K = 4570
+// 333.8 -> 41.4; M = 2, N = 832, K = 5908 83.1 -> 15.6; M = 4096, N = 512, K = 1000
+// 191.7 -> 27.3; fp16 M = 16, N = K = 258 37.1 -> 6.4. Tiny products keep the one
+// launch of the general kernel (M = 1, N = 20, K = 10: 5.4 against 5.8 us).
+template <int ACT>
+int w8a16_padded(const void* x, const int8_t* wq, const void* scales, const void* bias,
+                 const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N,
+                 int64_t K, void* ws, size_t ws_bytes, void* y, hipStream_t s) {
+  const int64_t kp = cdiv(K, 16LL) * 16;
+  const bool direct = pad_direct(M, N, K);
+  uint8_t* const xd = static_cast<uint8_t*>(ws) + CBQ_WS_CTRL_BYTES;
+  uint8_t* const wd = xd + pad_align(M * kp * 2);
+  PadArgs p{};
+  p.src[0] = static_cast<const uint8_t*>(x);
+  p.dst[0] = xd;
+  p.rows[0] = M;
+  p.kb[0] = K * 2;
+  p.ld[0] = kp * 2;
+  p.src[1] = reinterpret_cast<const uint8_t*>(wq);
+  p.dst[1] = wd;
+  p.rows[1] = direct ? 0 : N;
+  p.kb[1] = K;
+  p.ld[1] = kp;
+  launch_pad(p, s);
+  if (!direct) {
+    // the control block's offset before the partials, which nothing here reads
+    const int64_t used = pad_align(M * kp * 2) + pad_align(N * kp);
+    return w8a16_t<ACT>(xd, reinterpret_cast<const int8_t*>(wd), scales, bias, oc, n_out, w_out, M,
+                        N, kp, static_cast<uint8_t*>(ws) + used, ws_bytes - used, y, s);
+  }
+  GemmArgs a{};
+  a.x = static_cast<const uint16_t*>(x);
+  a.xp = reinterpret_cast<const uint16_t*>(xd);
+  a.ldx = static_cast<int>(kp);
+  a.wq = wq;
+  a.scales = static_cast<const uint16_t*>(scales);
+  a.bias = static_cast<const uint16_t*>(bias);
+  a.oc = oc;
+  a.w_out = static_cast<const uint16_t*>(w_out);
+  a.y = static_cast<uint16_t*>(y);
+  a.M = static_cast<int>(M);
+  a.N = static_cast<int>(N);
+  a.K = static_cast<int>(K);
+  a.n_out = static_cast<int>(n_out);
+  launch_decode<ACT>(a, s);
+  return launch_status("cbq_w8a16_linear");
+}
+
 template <int ACT>
 int w8a16_t(const void* x, const int8_t* wq, const void* scales, const void* bias,
             const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N, int64_t K,
             void* ws, size_t ws_bytes, void* y, hipStream_t s) {
+  if (pad_ok(M, N, K) && aligned(x, 2) && aligned(y, 8) && ws &&
+      ws_bytes >= static_cast<size_t>(CBQ_WS_CTRL_BYTES + pad_bytes(M, N, K)))
+    return w8a16_padded<ACT>(x, wq, scales, bias, oc, n_out, w_out, M, N, K, ws, ws_bytes, y, s);
   if (!mfma_path(M, N, K, x, wq, y))
     return w8a16_general<ACT>(x, wq, scales, bias, oc, n_out, w_out, M, N, K, ws, ws_bytes, y, s);
   GemmArgs a{};
@@ -2185,6 +2337,8 @@ int w8a16_t(const void* x, const int8_t* wq, const void* scales, const void* bia
   a.N = static_cast<int>(N);
   a.K = static_cast<int>(K);
   a.n_out = static_cast<int>(n_out);
+  a.xp = a.x;
+  a.ldx = a.K;
   DmaPlan plan{4, 0, 1};
   const Kind kind = choose(M, N, K, n_out, ws ? ws_bytes : 0, plan);
   if (kind == kTileDmaSplit)
@@ -2202,14 +2356,16 @@ extern "C" size_t cbq_w8a16_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t n_
                                      int act_dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return CBQ_WS_CTRL_BYTES;
   // fp16 / bf16 with K % 16 == 0 run the MFMA kernels (split-K partials of
-  // the last wave of tiles); fp32 and K % 16 != 0 run the general kernel
-  // (its partial sums). Unaligned fp16 / bf16 operands also take the general
+  // the last wave of tiles), K % 16 != 0 the same kernels on padded rows; fp32
+  // on the general kernel needs its partial sums. Unaligned fp16 / bf16 operands also take the general
   // kernel; with this size it then runs without a split (same results).
   const bool mfma = (act_dtype == kF16 || act_dtype == kBF16) && K % 16 == 0;
   const int64_t bytes =
       mfma ? splitk_bytes(M, N, split_plan(M, N, K))
       : (act_dtype == kF32 && f32lin::applies(M, N, K, n_out))
           ? std::max(f32lin::ws_bytes(M, N, K), general_split_bytes(M, N, K))
+      : (act_dtype != kF32 && pad_ok(M, N, K))
+          ? std::max(pad_bytes(M, N, K), general_split_bytes(M, N, K))
           : general_split_bytes(M, N, K);
   return CBQ_WS_CTRL_BYTES + static_cast<size_t>(bytes);
 }

@@ -246,7 +246,10 @@ int cbq_dequant_int8_group_nd(const int8_t* q, const float* scale,
 
 /* Workspace bytes for cbq_w8a16_linear at this shape and activation dtype:
  * the control block, plus the split-K scratch of the kernel that dtype
- * selects. CBQ_F16 / CBQ_BF16 with K % 16 == 0 (MFMA): for M > 64 when the
+ * selects. CBQ_F16 / CBQ_BF16 with K % 16 != 0: the rows of x, and unless M <=
+ * 32 with a weight of 8 MB or more those of the weight, padded to a multiple of
+ * 16, or the general kernel's partial sums if those are larger. CBQ_F16 /
+ * CBQ_BF16 (MFMA): for M > 64 when the
  * last wave of output tiles is short, the fp32 partial tiles of that wave
  * (ranges x tail tiles x 256 / 192 / 128 KiB for tiles of 256 / 192 / 128 x
  * 256; at most 16 ranges and at most one partial tile per CU, i.e. <= 64 MiB
@@ -257,7 +260,7 @@ int cbq_dequant_int8_group_nd(const int8_t* q, const float* scale,
  * per output and k-range (at most 16 and at most one tile per CU). A larger M
  * runs in chunks of rows (multiples of 256, one after another, reusing the
  * workspace) whose 4 M K bytes stay below 256 MiB. Other CBQ_F32
- * shapes and K % 16 != 0 (general kernel): fp32 partial sums, up to 16 x M x
+ * shapes (general kernel): fp32 partial sums, up to 16 x M x
  * N x 4 bytes when its tiles give fewer than two workgroups per CU. The
  * reference allocates its temporaries inside the forward (linear.py:105-131). */
 size_t cbq_w8a16_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t n_out, int act_dtype);
@@ -278,7 +281,8 @@ size_t cbq_w8a16_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t n_out, int ac
  * row of x as 24-bit fixed-point numbers against its largest magnitude, three
  * int8 digits multiplied exactly (elements above 128 times the row's mean
  * magnitude and non-finite ones are added in fp32); other CBQ_F32 calls,
- * K % 16 != 0 and unaligned operands run a tiled fp32-FMA kernel. K == 0
+ * unaligned operands and fp16 / bf16 with K % 16 != 0 and no room in ws for the
+ * padded rows run a tiled fp32-FMA kernel. K == 0
  * gives y = bias (or 0); x and wq may then be null.
  * wq: int8 [N,K] row-major; its outlier columns hold 0.
  * scales, bias (nullable): [N] act_dtype. outlier_cols: n_out int64 indices in
