@@ -46,14 +46,22 @@ def check_out_dtype(dtype: torch.dtype) -> int:
     return _abi.DTYPE_CODE[dtype]
 
 
-def check_exchange(dev: torch.device, what: str) -> None:
-    """With CUBLADE_CHECK_EXCHANGE=1 in the environment: synchronise after a
-    per-tensor quant and raise RuntimeError if its workgroups' exchange timed
-    out (the status word of the stream's workspace; cleared before raising).
-    Off by default, so that calls stay asynchronous; a timed-out call's scale
-    is NaN whenever a code is not exact, and later calls are exact either way."""
+def watch_exchange(dev: torch.device) -> bool:
+    """Whether CUBLADE_CHECK_EXCHANGE=1 is in the environment; if so, clears
+    the status word of the stream's workspace (in stream order), so that
+    check_exchange after the call tells of that call alone."""
     if os.environ.get("CUBLADE_CHECK_EXCHANGE", "") in ("", "0"):
-        return
+        return False
+    _abi.clear_tensor_quant_status(dev)
+    return True
+
+
+def check_exchange(dev: torch.device, what: str) -> None:
+    """Where watch_exchange returned True before a per-tensor quant:
+    synchronise after it and raise RuntimeError if its workgroups' exchange
+    timed out (the status word; cleared before raising). Off by default, so
+    that calls stay asynchronous; a timed-out call's scale is NaN whenever a
+    code is not exact, and later calls are exact either way."""
     if _abi.tensor_quant_status(dev):
         _abi.clear_tensor_quant_status(dev)
         raise RuntimeError(

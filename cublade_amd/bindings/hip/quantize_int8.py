@@ -5,7 +5,7 @@ from __future__ import annotations
 import torch
 
 from ... import _abi
-from ._common import check_exchange, check_float_input
+from ._common import check_exchange, check_float_input, watch_exchange
 
 
 def quantize_per_tensor_int8(
@@ -35,10 +35,12 @@ def quantize_per_tensor_int8(
     L = _abi.lib()
     with _abi.on_device(dev):
         ws = _abi.workspace(dev, L.cbq_quant_tensor_ws_bytes())
+        watch = watch_exchange(dev)
         rc = L.cbq_quant_int8_tensor(_abi.ptr(x), code, n, float(eps), _abi.ptr(ws), ws.numel(),
                                      _abi.ptr(q), _abi.ptr(scale), _abi.stream_handle(dev))
     _abi.check(rc, "quantize_per_tensor_int8")
-    check_exchange(dev, "quantize_per_tensor_int8")
+    if watch:
+        check_exchange(dev, "quantize_per_tensor_int8")
     return q, scale
 
 

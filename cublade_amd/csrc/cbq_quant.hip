@@ -14,8 +14,11 @@
 //                   written to the workspace (no atomics: measured on MI355X,
 //                   ~4k same-address device atomics cost ~100 us)
 //                   (quantize_per_tensor_fp8.cu:38-86, quantize_int8.cu:47-101)
+//   k_quant_tensor_small
+//                   the same for x up to 2^19 elements, one chunk of 8 elements
+//                   per thread (one workgroup of 4 per thread up to 2^15)
 //   k_cast_tensor   per-tensor cast on the same persistent grid (the two-pass
-//                   path for smaller or unaligned x): each workgroup
+//                   path for x between the two or unaligned): each workgroup
 //                   issues its first 16-byte loads, reduces the partial maxima
 //                   (L2-resident) to inv meanwhile, then 8-byte packed stores;
 //                   workgroup 0 writes the scale
@@ -623,17 +626,21 @@ __device__ __forceinline__ Raw8<DT> ld8_max(const unsigned long long* p, int64_t
 }
 
 // Waits until every slot [0, G) carries tag; after spin_limit polls
-// records suspect = tag and status = 1 (both performed before it) and polls
-// once more. Returns whether the wait completed (every thread gets it).
-__device__ int slot_wait(char* ctl, uint32_t tag, uint32_t spin_limit) {
+// records suspect = tag and, with REPORT, status = 1 (both performed before it)
+// and polls once more. Returns whether the wait completed (every thread gets it); mx:
+// the maximum of the values (as floats) of the slots this thread polled.
+template <bool REPORT>
+__device__ int slot_wait(char* ctl, uint32_t tag, uint32_t spin_limit, float& mx) {
   auto* slots = reinterpret_cast<unsigned long long*>(ctl + kCtlSlots);
   const int G = static_cast<int>(gridDim.x);
   auto poll = [&]() {
     int ok = 1;
+    mx = 0.0f;
     for (int i = threadIdx.x; i < G; i += blockDim.x) {
-      const uint32_t t = static_cast<uint32_t>(
-          __hip_atomic_load(slots + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32);
-      ok &= t == tag;
+      const unsigned long long v =
+          __hip_atomic_load(slots + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ok &= static_cast<uint32_t>(v >> 32) == tag;
+      mx = fmaxf(mx, __uint_as_float(static_cast<uint32_t>(v)));
     }
     return __syncthreads_and(ok);
   };
@@ -649,14 +656,32 @@ __device__ int slot_wait(char* ctl, uint32_t tag, uint32_t spin_limit) {
     if (threadIdx.x == 0) {
       __hip_atomic_store(reinterpret_cast<unsigned int*>(ctl + kCtlSuspect), tag, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(reinterpret_cast<unsigned int*>(ctl + kCtlStatus), 1u, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+      if (REPORT)
+        __hip_atomic_store(reinterpret_cast<unsigned int*>(ctl + kCtlStatus), 1u,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __builtin_amdgcn_s_waitcnt(0);
     }
     __syncthreads();
     ok = poll();
   }
   return ok;
+}
+
+// After a completed wait, by thread 0: workgroup 0, or any workgroup of a call
+// in which another gave up, makes tag the last call's; workgroup 0 also clears
+// an earlier call's record.
+__device__ __forceinline__ void advance_gen(char* ctl, uint32_t tag, int b) {
+  auto* gen_w = reinterpret_cast<unsigned long long*>(ctl + kCtlGen);
+  auto* suspect = reinterpret_cast<unsigned int*>(ctl + kCtlSuspect);
+  const uint32_t su = __hip_atomic_load(suspect, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (b == 0 || su == tag)
+    __hip_atomic_store(gen_w, static_cast<unsigned long long>(tag), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  if (b == 0 && su != 0 && su != tag) {
+    uint32_t expect = su;
+    __hip_atomic_compare_exchange_strong(suspect, &expect, 0u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // Thread 0 publishes the workgroup's slot with tag (after the workgroup's
@@ -841,20 +866,9 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_cols_strip(
     __syncthreads();
     const uint32_t tag = s_tag;
     slot_publish(ctl, tag, true);
-    const int ok = slot_wait(ctl, tag, spin_limit);
-    if (t == 0 && ok) {
-      auto* gen_w = reinterpret_cast<unsigned long long*>(ctl + kCtlGen);
-      auto* suspect = reinterpret_cast<unsigned int*>(ctl + kCtlSuspect);
-      const uint32_t su = __hip_atomic_load(suspect, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (b == 0 || su == tag)
-        __hip_atomic_store(gen_w, static_cast<unsigned long long>(tag), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      if (b == 0 && su != 0 && su != tag) {   // an earlier call's record
-        uint32_t expect = su;
-        __hip_atomic_compare_exchange_strong(suspect, &expect, 0u, __ATOMIC_RELAXED,
-                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
+    float unused;
+    const int ok = slot_wait<true>(ctl, tag, spin_limit, unused);
+    if (t == 0 && ok) advance_gen(ctl, tag, b);
     ColMax<DT> all;
     if (ok) {
       for (int p = tr; p < nrb; p += rps)
@@ -919,6 +933,94 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_cols_strip(
 #pragma unroll
     for (int u = 0; u < U; ++u) put(v[u], i * U + u);
   }
+}
+
+// ---------------------------------------------------------------------------
+// Per tensor in one launch for small x (16-byte aligned, up to 2^19
+// elements): U chunks per thread held in registers, one workgroup (U = 4, up to
+// 2^15 elements) or one per 1024 chunks (U = 1). Workgroups exchange their
+// maxima through the tagged slots of k_quant_tensor_1pass; one whose wait gives
+// up takes the maximum of all of x itself (at most 2 MB) and goes on, as in
+// k_quant_cols_strip, so every result is exact and there is nothing to report
+// in the status word. Bound: latency (one load, one
+// exchange). The second launch it saves cost 3.5 us of host time; GPU time of
+// bf16 to FP8 and back (amax + cast launches before): [16, 512] 6.9 -> 5.5 us,
+// [16, 2048] 7.7 -> 7.4, [16, 4096] .. [128, 4096] 7.8-8.0 -> 8.0-8.1. Slower
+// were: 2 chunks per thread ([128, 4096] fp32 6.9 -> 7.9), one workgroup above
+// 2^15, and the refresh of the unused slots before the wait.
+// ---------------------------------------------------------------------------
+template <int DT, bool FP8, int U>
+__global__ __launch_bounds__(kFusedBlock) void k_quant_tensor_small(
+    const void* __restrict__ x, int64_t n, float eps, uint8_t* __restrict__ q,
+    float* __restrict__ scale_out, char* __restrict__ ctl, uint32_t spin_limit) {
+  constexpr float kQ = FP8 ? kQmaxFp8 : kQmaxInt8;
+  __shared__ float red[kFusedBlock / kWave];
+  __shared__ uint32_t s_tag;
+  const int b = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
+  const int G = static_cast<int>(gridDim.x);
+  const int n8 = static_cast<int>(n >> 3);
+  auto* gen_w = reinterpret_cast<unsigned long long*>(ctl + kCtlGen);
+  auto* slots = reinterpret_cast<unsigned long long*>(ctl + kCtlSlots);
+  if (G > 1 && t == 0)
+    s_tag = next_tag(static_cast<uint32_t>(
+        __hip_atomic_load(gen_w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+  Raw8<DT> r[U];
+  float m = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = (b * U + u) * kFusedBlock + t;
+    if (c < n8) r[u] = ld8<DT>(x, static_cast<int64_t>(c) * 8);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if ((b * U + u) * kFusedBlock + t < n8) {
+      float f[8];
+      cvt8<DT>(r[u], f);
+      m = absmax8(f, m);
+    }
+  const int64_t te = static_cast<int64_t>(n8) * 8 + t;   // the < 8 trailing elements
+  const bool has_tail = b == 0 && t < 8 && te < n;
+  const float tail = has_tail ? ld1<DT>(x, te) : 0.0f;
+  m = block_max(fmaxf(m, __builtin_fabsf(tail)), red);
+  if (G > 1) {
+    const uint32_t tag = s_tag;
+    const unsigned long long mine =
+        (static_cast<unsigned long long>(tag) << 32) | __float_as_uint(m);
+    if (t == 0) {
+      __hip_atomic_store(slots + b, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __builtin_amdgcn_s_waitcnt(0);   // performed before any poll
+    }
+    float g;
+    const int ok = slot_wait<false>(ctl, tag, spin_limit, g);
+    if (ok) {
+      if (t == 0) advance_gen(ctl, tag, b);
+    } else {
+      g = 0.0f;
+      for (int c = t; c < n8; c += kFusedBlock) {
+        float f[8];
+        cvt8<DT>(ld8<DT>(x, static_cast<int64_t>(c) * 8), f);
+        g = absmax8(f, g);
+      }
+      if (t < 8 && te < n) g = fmaxf(g, __builtin_fabsf(ld1<DT>(x, te)));
+    }
+    m = block_max(g, red);
+  }
+  const float inv = inv_scale(m, eps, kQ);
+  if (b == 0 && t == 0) *scale_out = 1.0f / inv;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = (b * U + u) * kFusedBlock + t;
+    if (c < n8) {
+      float f[8];
+      cvt8<DT>(r[u], f);
+      stg8(q + static_cast<int64_t>(c) * 8, FP8 ? pack8_fp8(f, inv) : pack8_int8(f, inv));
+    }
+  }
+  if (has_tail) q[te] = FP8 ? q_fp8_1(tail * inv) : static_cast<uint8_t>(q_int8(tail * inv));
+  if (G > 1)   // slots beyond the grid: refreshed, never read (after the wait: off its path)
+    for (int k = t + 1; b + static_cast<int64_t>(k) * G < kMaxFusedGrid; k += kFusedBlock)
+      __hip_atomic_store(slots + b + k * G, static_cast<unsigned long long>(s_tag) << 32,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------
@@ -1915,6 +2017,13 @@ __global__ void k_clear_tensor_status(char* ctl) {
                      __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Elements up to which one workgroup does the whole tensor, and up to which one
+// chunk per thread does: from there to kFusedMinElems the two-pass path's 256-thread
+// workgroups use more CUs and take less GPU time ([255, 4096] bf16 to FP8 and
+// back 8.7 us against 9.0, fp32 to INT8 7.1 against 7.4).
+constexpr int64_t kSmallOneWg = 4 * 8 * kFusedBlock;
+constexpr int64_t kSmallElems = int64_t{1} << 19;
+
 template <int DT>
 int tensor_quant_t(const void* x, int64_t n, float eps, float* partial, char* ctl, uint8_t* q,
                    float* scale, bool fp8, hipStream_t s) {
@@ -1926,15 +2035,26 @@ int tensor_quant_t(const void* x, int64_t n, float eps, float* partial, char* ct
     // there are CUs (below 2^23 elements): the workgroups that would find no
     // chunk of x only lengthen the launch and the exchange. Measured on
     // MI355X (back-to-back launches): [1024, 4096] fp16 9.76 -> 8.67 us,
-    // [1024, 1024] bf16 FP8 9.10 -> 8.21 us. Below 2^20 elements the two-pass
-    // path's smaller workgroups spread a small x over more CUs: [16, 4096]
-    // bf16 FP8 6.5 us against 7.6 us for one 1024-thread workgroup.
+    // [1024, 1024] bf16 FP8 9.10 -> 8.21 us.
     const int64_t steps = cdiv(n >> 3, static_cast<int64_t>(kFusedBlock) * kFusedU);
     const dim3 g(static_cast<unsigned>(std::min<int64_t>(steps, device_cus()))), b(kFusedBlock);
     if (fp8)
       k_quant_tensor_1pass<DT, true><<<g, b, 0, s>>>(x, n, eps, q, scale, ctl, fused_spin_limit());
     else
       k_quant_tensor_1pass<DT, false><<<g, b, 0, s>>>(x, n, eps, q, scale, ctl, fused_spin_limit());
+    return launch_status(what);
+  }
+  if (vec && n <= kSmallElems) {
+    const dim3 b(kFusedBlock);
+    const uint32_t spin = std::min(fused_spin_limit(), kColsSpinLimit);
+    if (n <= kSmallOneWg) {
+      if (fp8) k_quant_tensor_small<DT, true, 4><<<dim3(1), b, 0, s>>>(x, n, eps, q, scale, ctl, spin);
+      else k_quant_tensor_small<DT, false, 4><<<dim3(1), b, 0, s>>>(x, n, eps, q, scale, ctl, spin);
+    } else {
+      const dim3 g(static_cast<unsigned>(cdiv(n >> 3, static_cast<int64_t>(kFusedBlock))));
+      if (fp8) k_quant_tensor_small<DT, true, 1><<<g, b, 0, s>>>(x, n, eps, q, scale, ctl, spin);
+      else k_quant_tensor_small<DT, false, 1><<<g, b, 0, s>>>(x, n, eps, q, scale, ctl, spin);
+    }
     return launch_status(what);
   }
   const int64_t grid = tensor_grid(n, vec);

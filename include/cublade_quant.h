@@ -58,9 +58,10 @@ enum { CBQ_OK = 0, CBQ_EINVAL = 1, CBQ_ELAUNCH = 2 };
  * NaN, INT8 codes 0 there); a scale that is not NaN comes with every code
  * exact. The next call on the workspace is exact again, with no reset; the
  * status word stays 1 until cbq_tensor_quant_status_clear. Per-column quant
- * (cbq_quant_int8_channel, axis 1) uses the block the same way, but a
- * workgroup that gives up there takes the maxima of its columns from x itself:
- * its results are exact either way, only the status word tells. The other
+ * (cbq_quant_int8_channel, axis 1) and per-tensor quant of at most 2^19
+ * elements use the block the same way, but a workgroup that gives up there
+ * takes the maxima from x itself, after a few milliseconds: the results are
+ * exact either way; the columns still set the status word. The other
  * entry points leave the control block alone. The rest is per-call scratch. One
  * workspace serves one stream at a time: calls that overlap in time must not
  * share it. */
