@@ -14,6 +14,15 @@ import torch
 from ... import _abi
 
 
+def out_like(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """An uninitialised contiguous tensor of x's shape and device (a plain
+    torch.Tensor also where x is of a subclass). empty_like takes 1.0 us of
+    host time, empty with a shape and a device 1.9."""
+    if type(x) is torch.Tensor:
+        return torch.empty_like(x, dtype=dtype, memory_format=torch.contiguous_format)
+    return torch.empty(x.shape, dtype=dtype, device=x.device)
+
+
 def check_cuda_contig(t: torch.Tensor, name: str) -> None:
     if not t.is_cuda:
         raise RuntimeError(f"{name} must be on CUDA")

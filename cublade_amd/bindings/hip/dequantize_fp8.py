@@ -5,7 +5,7 @@ from __future__ import annotations
 import torch
 
 from ... import _abi
-from ._common import check_cuda_contig, check_out_dtype, check_scale
+from ._common import check_cuda_contig, check_out_dtype, check_scale, out_like
 
 
 def dequantize_per_tensor_fp8(
@@ -28,7 +28,7 @@ def dequantize_per_tensor_fp8(
     if scale.numel() != 1:
         raise RuntimeError("scale must be a 0-d or 1-element tensor")
     out = check_out_dtype(dtype)
-    y = torch.empty(q.shape, dtype=dtype, device=q.device)
+    y = out_like(q, dtype)
     n = q.numel()
     if n == 0:
         return y

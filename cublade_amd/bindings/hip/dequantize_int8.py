@@ -2,10 +2,12 @@
 bindings/cuda/dequantize_int8.py:18-79, kernels/cuda/quantization/dequantize_int8.cu:210-273)."""
 from __future__ import annotations
 
+import operator
+
 import torch
 
 from ... import _abi
-from ._common import check_cuda_contig, check_out_dtype, check_scale
+from ._common import check_cuda_contig, check_out_dtype, check_scale, out_like
 
 
 def _check_q(q: torch.Tensor) -> None:
@@ -25,7 +27,7 @@ def dequantize_per_tensor_int8(
     out = check_out_dtype(dtype)
     if scale.numel() != 1:
         raise RuntimeError("scale must be a scalar for per-tensor mode")
-    y = torch.empty(q.shape, dtype=dtype, device=q.device)
+    y = out_like(q, dtype)
     n = q.numel()
     if n == 0:
         return y
@@ -58,7 +60,7 @@ def dequantize_per_channel_int8(
         raise RuntimeError("scale must have C elements (size(0) of q)")
     if axis == 1 and scale.numel() != F:
         raise RuntimeError("scale must have F elements (numel(q) / size(0)) for axis 1")
-    y = torch.empty(q.shape, dtype=dtype, device=q.device)
+    y = out_like(q, dtype)
     if C == 0 or F == 0:
         return y
     L = _abi.lib()
@@ -86,16 +88,38 @@ def dequantize_per_group_int8(
         raise RuntimeError("q_grouped.size(1) must equal group_size")
     if not (0 < group_size <= 4096):
         raise RuntimeError("group_size must be in (0, 4096]")
-    G = q_grouped.size(0)
+    return _dequant_groups(q_grouped, scale, q_grouped.size(0), group_size, dtype, out)
+
+
+def dequantize_groups_last_axis(
+    q: torch.Tensor,
+    scale: torch.Tensor,
+    group_size: int,
+    dtype: torch.dtype = torch.bfloat16,
+) -> torch.Tensor:
+    """dequantize_per_group_int8 of q.reshape(-1, group_size), in q's shape,
+    without views of q and the result (1 us of host time each)."""
+    _check_q(q)
+    scale = check_scale(scale, q)
+    out = check_out_dtype(dtype)
+    group_size = operator.index(group_size)
+    if not (0 < group_size <= 4096):
+        raise RuntimeError("group_size must be in (0, 4096]")
+    if q.numel() % group_size != 0:
+        raise RuntimeError(f"group_size {group_size} must evenly divide the {q.numel()} elements")
+    return _dequant_groups(q, scale, q.numel() // group_size, group_size, dtype, out)
+
+
+def _dequant_groups(q, scale, G: int, group_size: int, dtype, out: int) -> torch.Tensor:
     if scale.numel() != G:
         raise RuntimeError("scale must have num_groups elements")
-    y = torch.empty(q_grouped.shape, dtype=dtype, device=q_grouped.device)
+    y = out_like(q, dtype)
     if G == 0:
         return y
     L = _abi.lib()
-    with _abi.on_device(q_grouped.device):
-        rc = L.cbq_dequant_int8_group(_abi.ptr(q_grouped), _abi.ptr(scale), G, int(group_size),
-                                      _abi.ptr(y), out, _abi.stream_handle(q_grouped.device))
+    with _abi.on_device(q.device):
+        rc = L.cbq_dequant_int8_group(_abi.ptr(q), _abi.ptr(scale), G, int(group_size),
+                                      _abi.ptr(y), out, _abi.stream_handle(q.device))
     _abi.check(rc, "dequantize_per_group_int8")
     return y
 
@@ -120,7 +144,7 @@ def dequantize_per_channel_int8_nd(
     outer, C, inner = _axis_view(q.shape, axis)
     if scale.numel() != C:
         raise RuntimeError(f"scale must have {C} elements (size({axis}) of q)")
-    y = torch.empty(q.shape, dtype=dtype, device=q.device)
+    y = out_like(q, dtype)
     if q.numel() == 0:
         return y
     L = _abi.lib()
@@ -155,7 +179,7 @@ def dequantize_per_group_int8_nd(
     ng = outer * inner * (Lq // group_size)
     if scale.numel() != ng:
         raise RuntimeError(f"scale must have {ng} elements (one per group)")
-    y = torch.empty(q.shape, dtype=dtype, device=q.device)
+    y = out_like(q, dtype)
     if ng == 0:
         return y
     L = _abi.lib()

@@ -5,7 +5,7 @@ from __future__ import annotations
 import torch
 
 from ... import _abi
-from ._common import check_exchange, check_float_input, watch_exchange
+from ._common import check_exchange, check_float_input, out_like, watch_exchange
 
 
 def quantize_per_tensor_fp8(
@@ -30,7 +30,7 @@ def quantize_per_tensor_fp8(
     """
     code = check_float_input(x, allow_f32=False)
     dev = x.device
-    q = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=dev)
+    q = out_like(x, torch.float8_e4m3fn)
     n = x.numel()
     if n == 0:
         return q, torch.zeros((), dtype=torch.float32, device=dev)

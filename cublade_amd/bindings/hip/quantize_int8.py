@@ -2,10 +2,12 @@
 bindings/cuda/quantize_int8.py:18-87, kernels/cuda/quantization/quantize_int8.cu:470-536)."""
 from __future__ import annotations
 
+import operator
+
 import torch
 
 from ... import _abi
-from ._common import check_exchange, check_float_input, watch_exchange
+from ._common import check_exchange, check_float_input, out_like, watch_exchange
 
 
 def quantize_per_tensor_int8(
@@ -27,7 +29,7 @@ def quantize_per_tensor_int8(
     """
     code = check_float_input(x, allow_f32=True)
     dev = x.device
-    q = torch.empty(x.shape, dtype=torch.int8, device=dev)
+    q = out_like(x, torch.int8)
     n = x.numel()
     if n == 0:
         return q, torch.zeros((), dtype=torch.float32, device=dev)
@@ -67,7 +69,7 @@ def quantize_per_channel_int8(
     dev = x.device
     C = x.size(0)
     F = x.numel() // C if C else 0
-    q = torch.empty(x.shape, dtype=torch.int8, device=dev)
+    q = out_like(x, torch.int8)
     nscale = C if axis == 0 else F
     if C == 0 or F == 0:
         return q, torch.zeros((nscale,), dtype=torch.float32, device=dev)
@@ -97,15 +99,34 @@ def quantize_per_group_int8(
         raise RuntimeError("x_grouped.size(1) must equal group_size")
     if not (0 < group_size <= 4096):
         raise RuntimeError("group_size must be in (0, 4096]")
-    dev = x_grouped.device
-    G = x_grouped.size(0)
-    q = torch.empty(x_grouped.shape, dtype=torch.int8, device=dev)
+    return _quant_groups(x_grouped, code, x_grouped.size(0), group_size, eps)
+
+
+def quantize_groups_last_axis(
+    x: torch.Tensor,
+    group_size: int,
+    eps: float = 1e-12,
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """quantize_per_group_int8 of x.reshape(-1, group_size), with q in x's
+    shape: no views of x and q are made (1 us of host time each)."""
+    code = check_float_input(x, allow_f32=True)
+    group_size = operator.index(group_size)
+    if not (0 < group_size <= 4096):
+        raise RuntimeError("group_size must be in (0, 4096]")
+    if x.numel() % group_size != 0:
+        raise RuntimeError(f"group_size {group_size} must evenly divide the {x.numel()} elements")
+    return _quant_groups(x, code, x.numel() // group_size, group_size, eps)
+
+
+def _quant_groups(x, code: int, G: int, group_size: int, eps: float):
+    dev = x.device
+    q = out_like(x, torch.int8)
     if G == 0:
         return q, torch.zeros((0,), dtype=torch.float32, device=dev)
-    scale = torch.empty((G,), dtype=torch.float32, device=dev)
+    scale = torch.empty(G, dtype=torch.float32, device=dev)
     L = _abi.lib()
     with _abi.on_device(dev):
-        rc = L.cbq_quant_int8_group(_abi.ptr(x_grouped), code, G, int(group_size), float(eps),
+        rc = L.cbq_quant_int8_group(_abi.ptr(x), code, G, int(group_size), float(eps),
                                     _abi.ptr(q), _abi.ptr(scale), _abi.stream_handle(dev))
     _abi.check(rc, "quantize_per_group_int8")
     return q, scale
@@ -140,7 +161,7 @@ def quantize_per_channel_int8_nd(
         raise RuntimeError(f"axis {axis} out of range for a {x.dim()}-D tensor")
     dev = x.device
     outer, C, inner = _axis_view(x.shape, axis)
-    q = torch.empty(x.shape, dtype=torch.int8, device=dev)
+    q = out_like(x, torch.int8)
     if x.numel() == 0:
         return q, torch.zeros((C,), dtype=torch.float32, device=dev)
     scale = torch.empty((C,), dtype=torch.float32, device=dev)
@@ -175,7 +196,7 @@ def quantize_per_group_int8_nd(
     outer, Lx, inner = _axis_view(x.shape, axis)
     if Lx % group_size != 0:
         raise RuntimeError(f"group_size {group_size} must evenly divide axis length {Lx}")
-    q = torch.empty(x.shape, dtype=torch.int8, device=dev)
+    q = out_like(x, torch.int8)
     ng = outer * inner * (Lx // group_size)
     scale = torch.empty((ng,), dtype=torch.float32, device=dev)
     if ng == 0:

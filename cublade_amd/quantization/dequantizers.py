@@ -16,7 +16,7 @@ from cublade_amd.bindings.hip.dequantize_fp8 import (
 from cublade_amd.bindings.hip.dequantize_int8 import (
     dequantize_per_tensor_int8 as _hip_dequant_int8_tensor,
     dequantize_per_channel_int8 as _hip_dequant_int8_channel,
-    dequantize_per_group_int8 as _hip_dequant_int8_group,
+    dequantize_groups_last_axis as _hip_dequant_int8_group_last,
     dequantize_per_channel_int8_nd as _hip_dequant_int8_channel_nd,
     dequantize_per_group_int8_nd as _hip_dequant_int8_group_nd,
 )
@@ -74,9 +74,8 @@ def dequantize_tensor(qt: QuantizedTensor) -> torch.Tensor:
                     f"group_size {qt.group_size} must evenly divide axis length {F}"
                 )
             if q.dim() == 0 or ax == q.dim() - 1:
-                y_grouped = _hip_dequant_int8_group(q.reshape(-1, qt.group_size), qt.scale,
-                                                    qt.group_size, qt.original_dtype)
-                return y_grouped.view(q.shape)
+                return _hip_dequant_int8_group_last(q, qt.scale, qt.group_size,
+                                                    qt.original_dtype)
             # any other axis: strided groups, no movedim copies
             # (dequantizers.py:61-72 makes two full copies here)
             return _hip_dequant_int8_group_nd(q, qt.scale, ax, qt.group_size, qt.original_dtype)

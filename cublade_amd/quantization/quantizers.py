@@ -25,6 +25,7 @@ from cublade_amd.bindings.hip.quantize_int8 import (
     quantize_per_tensor_int8 as _hip_quant_int8_tensor,
     quantize_per_channel_int8 as _hip_quant_int8_channel,
     quantize_per_group_int8 as _hip_quant_int8_group,
+    quantize_groups_last_axis as _hip_quant_int8_group_last,
     quantize_per_channel_int8_nd as _hip_quant_int8_channel_nd,
     quantize_per_group_int8_nd as _hip_quant_int8_group_nd,
 )
@@ -146,8 +147,7 @@ def quantize_tensor(
             raise ValueError(f"group_size {group_size} must evenly divide axis length {F}")
         if x.dim() == 0 or ax == x.dim() - 1:
             # groups along the last axis are contiguous rows
-            q_grouped, scale = kernel(x.reshape(-1, group_size), group_size, eps)
-            q = q_grouped.view(x.shape)
+            q, scale = _hip_quant_int8_group_last(x, group_size, eps)
         else:
             # any other axis: strided groups, no movedim copies
             # (quantizers.py:123-132 makes two full copies here)
