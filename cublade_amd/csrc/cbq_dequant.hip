@@ -253,16 +253,17 @@ __global__ __launch_bounds__(kBlock) void k_deq_rows_scalar(
 }
 
 // Rows of any length L <= 2048 that 8-byte code loads cannot take (L % 8 !=
-// 0, e.g. groups of 100, or unaligned buffers): LPR lanes per row, VPL codes
-// per lane, code j = v * LPR + lr, loads and stores contiguous across the
-// lanes of a row.
+// 0, e.g. groups of 100, or unaligned buffers): LPR lanes per row, VPL units of
+// E codes per lane, unit j = v * LPR + lr, loads and stores contiguous across the
+// lanes of a row. E = 4 (L % 4 == 0, q and y aligned to a unit): one 4-byte load
+// and one 8-byte store; E = 2: pairs likewise. Bound: load and store
+// instructions; memory comes nearer with E = 4 (figures at k_rows_sub_any1, whose
+// layout this is).
 template <int OUT, int LPR, int VPL, int RI, int E>
 __global__ __launch_bounds__(kBlock) void k_deq_rows_sub_any1(
     const int8_t* __restrict__ q, const float* __restrict__ scale, int64_t rows, int L,
     void* __restrict__ y) {
-  // E = 2: code pairs (L even, q and y aligned to a pair): one 2-byte load
-  // and one 4-byte store per pair
-  static_assert(E == 1 || E == 2, "codes per load");
+  static_assert(E == 1 || E == 2 || E == 4, "codes per load");
   constexpr int RPW = kWave / LPR;
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
@@ -271,32 +272,48 @@ __global__ __launch_bounds__(kBlock) void k_deq_rows_sub_any1(
   const int U = L / E;
   const int64_t row0 =
       (static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + wave) * (RI * RPW) + sub;
+  uint32_t c[RI][VPL];   // every row's codes are in flight before the first is used
+  float sc[RI];
+#pragma unroll
+  for (int it = 0; it < RI; ++it) {
+    const int64_t row = row0 + static_cast<int64_t>(it) * RPW;
+    if (row < rows) {
+      sc[it] = scale[row];
+#pragma unroll
+      for (int v = 0; v < VPL; ++v) {
+        const int j = v * LPR + lr;
+        const int64_t e = row * L + static_cast<int64_t>(j < U ? j : 0) * E;
+        if constexpr (E == 1) c[it][v] = static_cast<uint8_t>(q[e]);
+        else if constexpr (E == 2) c[it][v] = *reinterpret_cast<const uint16_t*>(q + e);
+        else c[it][v] = *reinterpret_cast<const uint32_t*>(q + e);
+      }
+    }
+  }
 #pragma unroll
   for (int it = 0; it < RI; ++it) {
     const int64_t row = row0 + static_cast<int64_t>(it) * RPW;
     if (row >= rows) continue;
-    const float s = scale[row];
-    uint32_t c[VPL];
-#pragma unroll
-    for (int v = 0; v < VPL; ++v) {
-      const int j = v * LPR + lr;
-      const int64_t e = row * L + static_cast<int64_t>(j < U ? j : 0) * E;
-      if constexpr (E == 1) c[v] = static_cast<uint8_t>(q[e]);
-      else c[v] = *reinterpret_cast<const uint16_t*>(q + e);
-    }
+    const float s = sc[it];
 #pragma unroll
     for (int v = 0; v < VPL; ++v) {
       const int j = v * LPR + lr;
       if (j >= U) continue;
       const int64_t e = row * L + static_cast<int64_t>(j) * E;
-      const float a = static_cast<float>(static_cast<int8_t>(c[v] & 0xffu)) * s;
+      float f[4];
+      int8x4_to_f32(c[it][v], f);
+#pragma unroll
+      for (int k = 0; k < E; ++k) f[k] *= s;
       if constexpr (E == 1) {
-        st1<OUT>(y, e, a);
+        st1<OUT>(y, e, f[0]);
       } else {
-        float b = static_cast<float>(static_cast<int8_t>((c[v] >> 8) & 0xffu)) * s;
-        float a2 = a;
-        asm volatile("" : "+v"(a2), "+v"(b));   // finished fp32 products, as in out1
-        *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(y) + e) = pack2_out<OUT>(a2, b);
+        asm volatile("" : "+v"(f[0]), "+v"(f[1]));   // finished fp32 products, as in out1
+        if constexpr (E == 2) {
+          *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(y) + e) = pack2_out<OUT>(f[0], f[1]);
+        } else {
+          asm volatile("" : "+v"(f[2]), "+v"(f[3]));
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + e) =
+              make_uint2(pack2_out<OUT>(f[0], f[1]), pack2_out<OUT>(f[2], f[3]));
+        }
       }
     }
   }
@@ -586,11 +603,19 @@ void deq_rows_any(const int8_t* q, const float* scale, int64_t rows, int cg, voi
 template <int OUT, int LPR, int VPL, int E>
 void launch_deq_rows_sub_any1(const int8_t* q, const float* scale, int64_t rows, int L, void* y,
                               hipStream_t s) {
-  constexpr int RI = VPL >= 16 ? 1 : 2;
-  constexpr int64_t rows_per_wg = static_cast<int64_t>(kBlock / kWave) * RI * (kWave / LPR);
-  k_deq_rows_sub_any1<OUT, LPR, VPL, RI, E>
-      <<<dim3(static_cast<unsigned>(cdiv(rows, rows_per_wg))), dim3(kBlock), 0, s>>>(q, scale,
-                                                                                     rows, L, y);
+  // rows per wave and lane group: with E = 4 and one unit per lane four where
+  // that leaves two workgroups per CU, else one (see k_rows_sub_any1's launch)
+  constexpr int kRows = E == 4 ? (VPL >= 4 ? 1 : VPL == 2 ? 2 : 4) : VPL >= 16 ? 1 : 2;
+  constexpr int64_t kPer = static_cast<int64_t>(kBlock / kWave) * (kWave / LPR);
+  if constexpr (kRows == 4) {
+    if (cdiv(rows, kPer * kRows) < 2LL * device_cus()) {
+      k_deq_rows_sub_any1<OUT, LPR, VPL, 1, E>
+          <<<dim3(static_cast<unsigned>(cdiv(rows, kPer))), dim3(kBlock), 0, s>>>(q, scale, rows, L, y);
+      return;
+    }
+  }
+  k_deq_rows_sub_any1<OUT, LPR, VPL, kRows, E>
+      <<<dim3(static_cast<unsigned>(cdiv(rows, kPer * kRows))), dim3(kBlock), 0, s>>>(q, scale, rows, L, y);
 }
 
 template <int OUT, int E>
@@ -607,13 +632,15 @@ void deq_rows_any1_e(const int8_t* q, const float* scale, int64_t rows, int L, v
   else if (U <= 128) launch_deq_rows_sub_any1<OUT, 64, 2, E>(q, scale, rows, L, y, s);
   else if (U <= 256) launch_deq_rows_sub_any1<OUT, 64, 4, E>(q, scale, rows, L, y, s);
   else if (U <= 512) launch_deq_rows_sub_any1<OUT, 64, 8, E>(q, scale, rows, L, y, s);
-  else launch_deq_rows_sub_any1<OUT, 64, 16, E>(q, scale, rows, L, y, s);
+  else if constexpr (E < 4) launch_deq_rows_sub_any1<OUT, 64, 16, E>(q, scale, rows, L, y, s);
 }
 
 template <int OUT>
 void deq_rows_any1(const int8_t* q, const float* scale, int64_t rows, int L, void* y,
                    hipStream_t s) {
-  if (L % 2 == 0 && aligned(q, 2) && aligned(y, 4))
+  if (L % 4 == 0 && aligned(q, 4) && aligned(y, 8))   // L <= 2048: U <= 512
+    deq_rows_any1_e<OUT, 4>(q, scale, rows, L, y, s);
+  else if (L % 2 == 0 && aligned(q, 2) && aligned(y, 4))
     deq_rows_any1_e<OUT, 2>(q, scale, rows, L, y, s);
   else if (L <= 1024)
     deq_rows_any1_e<OUT, 1>(q, scale, rows, L, y, s);

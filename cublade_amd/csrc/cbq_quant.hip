@@ -1133,18 +1133,33 @@ __global__ __launch_bounds__(kBlock) void k_rows_sub_any(
   }
 }
 
+// Two 16-bit elements of one word as floats.
+template <int DT>
+__device__ __forceinline__ void pair_f32(uint32_t w, float* f) {
+  if constexpr (DT == kBF16) {
+    f[0] = __uint_as_float(w << 16);
+    f[1] = __uint_as_float(w & 0xffff0000u);
+  } else {
+    f[0] = static_cast<float>(__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu)));
+    f[1] = static_cast<float>(__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)));
+  }
+}
+
 // Rows (groups) of any length L <= 2048 that 16-byte loads cannot take (L %
 // 8 != 0, e.g. groups of 100, or unaligned buffers): LPR lanes per row, VPL
-// elements per lane, element j = v * LPR + lr, 2- or 4-byte loads that are
-// contiguous across the lanes of a row. Slots past L load the row's first
-// element, stay out of the maximum and store nothing.
+// load units of E elements per lane, unit j = v * LPR + lr, contiguous across the
+// lanes of a row. Slots past L load the row's first unit, stay out of the
+// maximum and store nothing. E = 4 (L % 4 == 0, x and q aligned to a unit): one
+// 8-byte load (16 for fp32) and one 4-byte code store; E = 2: pairs likewise.
+// Bound: load and store instructions; memory comes nearer with E = 4. Quant and
+// dequant pass in groups of 100, E = 2 -> 4: bf16 [8192, 8000] 146 -> 85 us, fp16
+// [4099, 1400] 16.9 -> 12.8; rows of 1004 [8000, 1004] 15.0 -> 13.1; fp32 quant
+// [8192, 8000] 111 -> 64.
 template <int DT, int LPR, int VPL, int RI, int E>
 __global__ __launch_bounds__(kBlock) void k_rows_sub_any1(
     const void* __restrict__ x, int64_t rows, int L, float eps, int8_t* __restrict__ q,
     float* __restrict__ scale) {
-  // E = 2: element pairs (L even, x and q aligned to a pair) in one load and
-  // one 2-byte code store
-  static_assert(E == 1 || E == 2, "elements per load");
+  static_assert(E == 1 || E == 2 || E == 4, "elements per load");
   constexpr int RPW = kWave / LPR;
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
@@ -1165,19 +1180,23 @@ __global__ __launch_bounds__(kBlock) void k_rows_sub_any1(
         const int64_t e = row * L + static_cast<int64_t>(j < U ? j : 0) * E;
         if constexpr (E == 1) {
           f[it][v][0] = ld1<DT>(x, e);
+        } else if constexpr (E == 4 && DT == kF32) {
+          const float4 w = *reinterpret_cast<const float4*>(static_cast<const float*>(x) + e);
+          f[it][v][0] = w.x;
+          f[it][v][1] = w.y;
+          f[it][v][2] = w.z;
+          f[it][v][3] = w.w;
+        } else if constexpr (E == 4) {
+          const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(x) + e);
+          pair_f32<DT>(w.x, f[it][v]);
+          pair_f32<DT>(w.y, f[it][v] + 2);
         } else if constexpr (DT == kF32) {
           const float2 w = *reinterpret_cast<const float2*>(static_cast<const float*>(x) + e);
           f[it][v][0] = w.x;
           f[it][v][1] = w.y;
         } else {
           const uint32_t w = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(x) + e);
-          if constexpr (DT == kBF16) {
-            f[it][v][0] = __uint_as_float(w << 16);
-            f[it][v][1] = __uint_as_float(w & 0xffff0000u);
-          } else {
-            f[it][v][0] = static_cast<float>(__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu)));
-            f[it][v][1] = static_cast<float>(__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)));
-          }
+          pair_f32<DT>(w, f[it][v]);
         }
       }
     }
@@ -1191,7 +1210,8 @@ __global__ __launch_bounds__(kBlock) void k_rows_sub_any1(
 #pragma unroll
       for (int v = 0; v < VPL; ++v) {
         float mv = __builtin_fabsf(f[it][v][0]);
-        if constexpr (E == 2) mv = fmaxf(mv, __builtin_fabsf(f[it][v][1]));
+#pragma unroll
+        for (int k = 1; k < E; ++k) mv = fmaxf(mv, __builtin_fabsf(f[it][v][k]));
         m = v * LPR + lr < U ? fmaxf(m, mv) : m;
       }
     }
@@ -1204,6 +1224,10 @@ __global__ __launch_bounds__(kBlock) void k_rows_sub_any1(
         if (j < U) {
           if constexpr (E == 1) {
             q[row * L + j] = static_cast<int8_t>(q_int8(f[it][v][0] * inv));
+          } else if constexpr (E == 4) {
+            *reinterpret_cast<uint32_t*>(q + row * L + static_cast<int64_t>(j) * 4) =
+                pack4_low_bytes(q_int8(f[it][v][0] * inv), q_int8(f[it][v][1] * inv),
+                                q_int8(f[it][v][2] * inv), q_int8(f[it][v][3] * inv));
           } else {
             const uint32_t c0 = static_cast<uint8_t>(q_int8(f[it][v][0] * inv));
             const uint32_t c1 = static_cast<uint8_t>(q_int8(f[it][v][1] * inv));
@@ -2183,10 +2207,21 @@ void rows_quant_any(const void* x, int64_t rows, int cg, float eps, int8_t* q, f
 template <int DT, int LPR, int VPL, int E>
 void launch_rows_sub_any1(const void* x, int64_t rows, int L, float eps, int8_t* q, float* scale,
                           hipStream_t s) {
-  constexpr int RI = VPL >= 16 ? 1 : 2;
-  constexpr int64_t rows_per_wg = static_cast<int64_t>(kBlock / kWave) * RI * (kWave / LPR);
-  k_rows_sub_any1<DT, LPR, VPL, RI, E><<<dim3(static_cast<unsigned>(cdiv(rows, rows_per_wg))),
-                                         dim3(kBlock), 0, s>>>(x, rows, L, eps, q, scale);
+  // rows per wave and lane group: with E = 4 and one unit per lane four where
+  // that leaves two workgroups per CU, else one (a group quant and dequant pass,
+  // fp16: [4099, 1400] in groups of 100 12.8 us; [500,
+  // 700] 4.9 with one, 5.8 with four)
+  constexpr int kRows = E == 4 ? (VPL >= 4 ? 1 : VPL == 2 ? 2 : 4) : VPL >= 16 ? 1 : 2;
+  constexpr int64_t kPer = static_cast<int64_t>(kBlock / kWave) * (kWave / LPR);
+  if constexpr (kRows == 4) {
+    if (cdiv(rows, kPer * kRows) < 2LL * device_cus()) {
+      k_rows_sub_any1<DT, LPR, VPL, 1, E>
+          <<<dim3(static_cast<unsigned>(cdiv(rows, kPer))), dim3(kBlock), 0, s>>>(x, rows, L, eps, q, scale);
+      return;
+    }
+  }
+  k_rows_sub_any1<DT, LPR, VPL, kRows, E>
+      <<<dim3(static_cast<unsigned>(cdiv(rows, kPer * kRows))), dim3(kBlock), 0, s>>>(x, rows, L, eps, q, scale);
 }
 
 constexpr int kRowsAny1Max = 2048;
@@ -2205,14 +2240,16 @@ void rows_quant_any1_e(const void* x, int64_t rows, int L, float eps, int8_t* q,
   else if (U <= 128) launch_rows_sub_any1<DT, 64, 2, E>(x, rows, L, eps, q, scale, s);
   else if (U <= 256) launch_rows_sub_any1<DT, 64, 4, E>(x, rows, L, eps, q, scale, s);
   else if (U <= 512) launch_rows_sub_any1<DT, 64, 8, E>(x, rows, L, eps, q, scale, s);
-  else launch_rows_sub_any1<DT, 64, 16, E>(x, rows, L, eps, q, scale, s);
+  else if constexpr (E < 4) launch_rows_sub_any1<DT, 64, 16, E>(x, rows, L, eps, q, scale, s);
 }
 
 template <int DT>
 void rows_quant_any1(const void* x, int64_t rows, int L, float eps, int8_t* q, float* scale,
                      hipStream_t s) {
   constexpr uintptr_t pair = DT == kF32 ? 8 : 4;
-  if (L % 2 == 0 && aligned(x, pair) && aligned(q, 2))
+  if (L % 4 == 0 && aligned(x, 2 * pair) && aligned(q, 4))   // L <= 2048: U <= 512
+    rows_quant_any1_e<DT, 4>(x, rows, L, eps, q, scale, s);
+  else if (L % 2 == 0 && aligned(x, pair) && aligned(q, 2))
     rows_quant_any1_e<DT, 2>(x, rows, L, eps, q, scale, s);
   else if (L <= 1024)
     rows_quant_any1_e<DT, 1>(x, rows, L, eps, q, scale, s);
