@@ -8,8 +8,6 @@
 namespace cbq {
 namespace f32lin {
 
-constexpr int kMaxSeg = 16384;   // k per row scale (see cbq_w8a16_f32.hip)
-
 // Whether the path takes a call (operands 16-byte aligned besides): no outlier
 // columns, K % 64 == 0, 32-bit operand offsets, and M > 64 or a weight of at
 // least 8 MB (below that the general kernel's single launch is as fast).

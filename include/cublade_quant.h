@@ -255,12 +255,11 @@ int cbq_dequant_int8_group_nd(const int8_t* q, const float* scale,
  * (ranges x tail tiles x 256 / 192 / 128 KiB for tiles of 256 / 192 / 128 x
  * 256; at most 16 ranges and at most one partial tile per CU, i.e. <= 64 MiB
  * on MI355X; the same with outlier columns), else nothing. CBQ_F32 on the
- * matrix-core path (see cbq_w8a16_linear): three int8 digit planes of x
- * (3 M K bytes; the size is never below 4 M K), 520 bytes per row of scales
- * and spike lists (per k-range above K = 16384) and, when K is split, 4 bytes
- * per output and k-range (at most 16 and at most one tile per CU). A larger M
- * runs in chunks of rows (multiples of 256, one after another, reusing the
- * workspace) whose 4 M K bytes stay below 256 MiB. Other CBQ_F32
+ * matrix-core path (see cbq_w8a16_linear): two 16-bit planes of x (4 M K
+ * bytes), 4 bytes per row and, when K is split, 4 bytes per output and
+ * k-range (at most 16 and at most one tile per CU). A larger M runs in chunks
+ * of rows (multiples of 256, one after another, reusing the workspace) whose
+ * planes stay within 192 MiB (or of 256 rows where those alone exceed it). Other CBQ_F32
  * shapes (general kernel): fp32 partial sums, up to 16 x M x
  * N x 4 bytes when its tiles give fewer than two workgroups per CU. The
  * reference allocates its temporaries inside the forward (linear.py:105-131). */
@@ -278,10 +277,11 @@ size_t cbq_w8a16_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t n_out, int ac
  * x: [M,K] and y: [M,N] in act_dtype, row-major. CBQ_F16 / CBQ_BF16 run
  * on MFMA. CBQ_F32 (the reference's fp32 Triton path, TF32 precision on its
  * hardware) with K % 64 == 0, no outlier columns, M > 64 or a weight of at
- * least 8 MB, and a workspace of cbq_w8a16_ws_bytes also runs on MFMA: each
- * row of x as 24-bit fixed-point numbers against its largest magnitude, three
- * int8 digits multiplied exactly (elements above 128 times the row's mean
- * magnitude and non-finite ones are added in fp32); other CBQ_F32 calls,
+ * least 8 MB, and a workspace of cbq_w8a16_ws_bytes also runs on MFMA: x as two
+ * fp16 planes under a power-of-two scale per row, 16 to 22 significant bits of
+ * every element (rows whose non-zero magnitudes span more than 2^34 as three
+ * bf16 numbers instead, exact, at up to 2.5 times the time), fp32
+ * accumulation; other CBQ_F32 calls,
  * unaligned operands and fp16 / bf16 with K % 16 != 0 and no room in ws for the
  * padded rows run a tiled fp32-FMA kernel. K == 0
  * gives y = bias (or 0); x and wq may then be null.

@@ -3,7 +3,7 @@ against the oracle's exact-accumulation W8A16 (float64) and the golden
 vectors. Gate (north star): rtol 1e-2 / atol 1e-2.
 
 Covers the MFMA path (fp16 / bf16, M / N / K tails), fp32 activations on the
-matrix cores as int8 digits (M > 64, K % 64 == 0), the general path (other
+matrix cores as two fp16 planes (M > 64, K % 64 == 0), the general path (other
 fp32 shapes, K not a multiple of 16, unaligned activations), bias, the
 outlier side-GEMM, quantize_model on an MLP, state_dict round trips (own and
 reference compact layout) and the BASELINE config-5 shapes (row subsets
@@ -164,11 +164,11 @@ def test_general_path_fp32_tiles(M, K, N):
 def test_fp32_two_plane_path(M, K, N):
     """fp32 activations with K % 64 == 0, no outlier columns and M > 64 (or
     M <= 64 with a weight of at least 8 MB; K may be split into
-    ranges) run on the matrix cores as int8 digits of x against the int8
+    ranges) run on the matrix cores as two 16-bit planes of x against the int8
     weights. Sampled rows
     against the oracle; the whole output against a float64 product within
-    2^-14 of sum_k |x w s| (one digit less would leave 16 bits against the
-    row's largest element); with outlier columns the VALU kernel runs, also
+    2^-14 of sum_k |x w s| (x keeps at least 16 significant bits; one plane
+    would leave 11); with outlier columns the VALU kernel runs, also
     against the oracle."""
     from cublade_amd import _abi
     assert _abi.lib().cbq_w8a16_ws_bytes(M, N, K, 0, _abi.DTYPE_CODE[torch.float32]) > \

@@ -103,12 +103,11 @@ def test_workspace_sizes():
     assert big >= C + 8192 * 4 * 2 and big < 64 << 20
     F16, F32 = _abi.F16, _abi.F32
     # M <= 16, fp16: the weight-streaming kernel, no partials. fp32 activations:
-    # the larger of the two-plane path's needs (two bf16 planes of x, then 2
-    # planes x 2 k-ranges x 43 tiles of 128 x 256 fp32 partials) and the
-    # general kernel's (16 k-ranges of [16, 11008] fp32 partial sums)
+    # the larger of the matrix-core path's needs (two 16-bit planes of x, 4 bytes
+    # per row, fp32 sums of the k-ranges) and the general kernel's (16 k-ranges of
+    # [16, 11008] fp32 partial sums)
     assert L.cbq_w8a16_ws_bytes(16, 11008, 4096, 0, F16) == C
-    planes16 = 2 * 16 * 4096 * 2 + 2 * 2 * 43 * 128 * 256 * 4
-    assert L.cbq_w8a16_ws_bytes(16, 11008, 4096, 0, F32) == C + max(planes16, 16 * 16 * 11008 * 4)
+    assert L.cbq_w8a16_ws_bytes(16, 11008, 4096, 0, F32) == C + 16 * 16 * 11008 * 4
     # a weight under 8 MB keeps the general kernel at M <= 64
     assert L.cbq_w8a16_ws_bytes(16, 1024, 4096, 0, F32) == C + 16 * 16 * 1024 * 4
     assert L.cbq_w8a16_ws_bytes(4096, 11008, 4096, 0, F16) == C
@@ -129,13 +128,14 @@ def test_workspace_sizes():
     # 24 < M <= 64 with K > 8192: the split MFMA path (11 ranges x 16 tiles of 128 x 256)
     assert L.cbq_w8a16_ws_bytes(64, 4096, 11008, 0, F16) == C + 11 * 16 * 128 * 1024
     assert L.cbq_w8a16_ws_bytes(32, 4096, 11008, 0, F16) == C + 11 * 16 * 128 * 1024
-    # M = 24: k_stream<2>, no MFMA partials; fp32: the two-plane path (bf16
-    # planes, then 2 planes x 8 k-ranges x 16 tiles of 128 x 256 fp32), larger
-    # than the general kernel's 16 ranges of [24, 4096] fp32
+    # M = 24: k_stream<2>, no MFMA partials; fp32: the general kernel's 16 ranges of
+    # [24, 4096] fp32 again; M = 500: whole tiles, the planes and row exponents alone;
+    # rows past 192 MiB of planes in chunks (12288 rows at K = 4096)
     assert L.cbq_w8a16_ws_bytes(24, 4096, 11008, 0, F16) == C
-    planes24 = 2 * 24 * 11008 * 2 + 2 * 8 * 16 * 128 * 256 * 4
-    assert planes24 > 16 * 24 * 4096 * 4
-    assert L.cbq_w8a16_ws_bytes(24, 4096, 11008, 0, F32) == C + planes24
+    assert L.cbq_w8a16_ws_bytes(24, 4096, 11008, 0, F32) == C + 16 * 24 * 4096 * 4
+    assert L.cbq_w8a16_ws_bytes(500, 11008, 4096, 0, F32) == C + 500 * 4096 * 4 + 2048
+    assert L.cbq_w8a16_ws_bytes(100000, 11008, 4096, 0, F32) == C + 12288 * (4096 * 4 + 4)
+    assert L.cbq_w8a16_ws_bytes(1 << 20, 256, 64, 0, F32) <= C + (204 << 20)
     # K % 16 != 0 takes the general kernel whatever the dtype
     assert L.cbq_w8a16_ws_bytes(16, 11008, 4090, 0, F16) == L.cbq_w8a16_ws_bytes(
         16, 11008, 4090, 0, F32)
