@@ -146,8 +146,13 @@ def quantize_tensor(
         if F % group_size != 0:
             raise ValueError(f"group_size {group_size} must evenly divide axis length {F}")
         if x.dim() == 0 or ax == x.dim() - 1:
-            # groups along the last axis are contiguous rows
-            q, scale = _hip_quant_int8_group_last(x, group_size, eps)
+            # groups along the last axis are contiguous rows; the registered kernel
+            # takes them as a 2-D view, its own binding also without one
+            if kernel is _hip_quant_int8_group:
+                q, scale = _hip_quant_int8_group_last(x, group_size, eps)
+            else:
+                q_grouped, scale = kernel(x.reshape(-1, group_size), group_size, eps)
+                q = q_grouped.view(x.shape)
         else:
             # any other axis: strided groups, no movedim copies
             # (quantizers.py:123-132 makes two full copies here)

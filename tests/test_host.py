@@ -485,3 +485,24 @@ def test_benchmark_returns_the_reference_contract(capsys):
     assert res["kernel"]["time_ms"] > 0 and res["reference"]["gflops"] > 0
     out = capsys.readouterr().out
     assert "GFLOPS" in out and "PASS" in out and "REF" in out
+
+
+def test_registered_group_kernel_is_called(monkeypatch):
+    """A kernel put in the registry in place of the library's is the one that
+    quantizes groups along the last axis (a CPU stand-in; no device work)."""
+    import torch
+
+    from cublade_amd.quantization import quantizers as Q
+
+    calls = []
+
+    def kernel(x_grouped, group_size, eps):
+        calls.append((tuple(x_grouped.shape), group_size, eps))
+        return torch.ones_like(x_grouped, dtype=torch.int8), torch.ones(x_grouped.size(0))
+
+    monkeypatch.setitem(Q._HIP_QUANT_KERNELS, ("group", torch.int8), kernel)
+    monkeypatch.setattr(Q, "_require_cuda_input", lambda x, key, *, what: None)
+    monkeypatch.setattr(Q, "_zero_scalar", lambda device: torch.zeros(()))
+    qt = Q.quantize_tensor(torch.randn(3, 4, 64), mode="group", group_size=32, ch_axis=-1, eps=1e-6)
+    assert calls == [((24, 32), 32, 1e-6)]
+    assert qt.data.shape == (3, 4, 64) and bool((qt.data == 1).all()) and qt.scale.shape == (24,)
