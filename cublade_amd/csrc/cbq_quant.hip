@@ -557,12 +557,12 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_tensor_1pass(
 //
 // Tags follow the per-tensor exchange (the same control block: gen, status,
 // suspect, slots; one tag per call). A workgroup whose wait gives up does not
-// need the others: it takes the maxima of its strip from x itself and goes
-// on, so every result is exact however the workgroups are scheduled (two
-// such grids on two streams may each hold some of the CUs); it still sets
-// status, and suspect so that a workgroup that completes advances gen (the
-// last workgroup to publish always completes). Waits are therefore short:
-// kColsSpinLimit polls at most.
+// need the others: it takes the maxima of the row blocks that are missing from x
+// itself and goes on, so every result is exact however the workgroups are
+// scheduled (other work may hold CUs for longer than the call takes); it still
+// sets status, and suspect so that a workgroup that completes advances gen (the
+// last workgroup to publish always completes). Waits are therefore short, see
+// short_spin_limit.
 // ---------------------------------------------------------------------------
 constexpr int kColsMaxSL = 6;                     // strips of at most 64 chunks
 // Chunks in flight per thread (64 bytes), steps of that many held in
@@ -571,7 +571,6 @@ constexpr int kColsMaxSL = 6;                     // strips of at most 64 chunks
 template <int DT> constexpr int strip_u() { return DT == kF32 ? 2 : 4; }
 template <int DT> constexpr int strip_hold() { return DT == kF32 ? 5 : 6; }
 constexpr int kStripPark = 2;
-constexpr uint32_t kColsSpinLimit = 4096;         // polls, a few milliseconds
 // Largest x (bytes) of the one-launch column path; larger ones take
 // k_colmax + k_cast_cols. A compile-time tuning knob.
 #ifndef CBQ_COLS_1PASS_MAX_BYTES
@@ -779,6 +778,7 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_cols_strip(
   constexpr int NP = max_planes<DT>();
   __shared__ u32x4 park[LS * U * QW * kFusedBlock];
   __shared__ unsigned int smax[2][8 << kColsMaxSL];   // [8 columns of a chunk][SW], as float bits
+  __shared__ uint8_t s_there[kMaxFusedGrid];
   __shared__ uint32_t s_tag;
 
   const int b = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
@@ -869,14 +869,28 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_cols_strip(
     float unused;
     const int ok = slot_wait<true>(ctl, tag, spin_limit, unused);
     if (t == 0 && ok) advance_gen(ctl, tag, b);
+    // Which row blocks to take from part: all, or after giving up those whose slot
+    // is there by now (decided once for the workgroup); the others' rows from x.
+    if (!ok) {
+      auto* slots = reinterpret_cast<unsigned long long*>(ctl + kCtlSlots);
+      for (int p = t; p < nrb; p += kFusedBlock)
+        s_there[p] = static_cast<uint32_t>(__hip_atomic_load(slots + p * strips + strip, __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT) >> 32) == tag;
+      __syncthreads();
+    }
     ColMax<DT> all;
-    if (ok) {
-      for (int p = tr; p < nrb; p += rps)
-        all.add(ld8_max<DT>(sp + static_cast<int64_t>(p) * NP * SW, SW, cc));
-    } else if (col_ok) {
-      // gave up waiting: the strip's maxima from x itself
+    for (int p = tr; p < nrb; p += rps)
+      if (ok || s_there[p]) all.add(ld8_max<DT>(sp + static_cast<int64_t>(p) * NP * SW, SW, cc));
+    if (!ok && col_ok) {
       const int64_t c0 = (static_cast<int64_t>(strip) * SW + cc) * 8;
-      for (int64_t rr = tr; rr < rows; rr += rps) all.add(ld8<DT>(x, rr * c8 * 8 + c0));
+      for (int p = 0; p < nrb; ++p)
+        if (!s_there[p])
+          for (int64_t rr = p * RB + tr, re = min((p + 1) * RB, rows); rr < re; rr += 2 * rps) {
+            const Raw8<DT> v0 = ld8<DT>(x, rr * c8 * 8 + c0);   // two: more would spill
+            const Raw8<DT> v1 = ld8<DT>(x, min(rr + rps, re - 1) * c8 * 8 + c0);
+            all.add(v0);
+            all.add(v1);
+          }
     }
     all.across(SW);
     if (t % kWave < SW) {
@@ -2018,6 +2032,16 @@ std::atomic<uint32_t>& spin_limit_var() {
 }
 uint32_t fused_spin_limit() { return spin_limit_var().load(std::memory_order_relaxed); }
 
+// The same where a workgroup that gives up can do without the others: polls (0.6 us
+// each) for x of so many bytes. A workgroup with little to read waits for about the
+// time that x takes to be read (0.2 us per MiB, a third of a poll). With these limits
+// none of 100 uncontended calls gave up at any of 15 shapes up to 480 MiB; bf16
+// [11008, 4096] beside a kernel that holds 32 CUs for 8 ms takes 144 us (with 4096
+// polls and the whole strip again 2300-2600; alone 29, as three launches 48).
+uint32_t short_spin_limit(int64_t bytes) {
+  return std::min(fused_spin_limit(), 64u + static_cast<uint32_t>(bytes >> 21));
+}
+
 // True if one workgroup of the one-launch kernel fits on a CU, i.e. a grid
 // of one workgroup per CU is resident at once (cached per device and kernel).
 template <int DT, bool FP8>
@@ -2070,7 +2094,7 @@ int tensor_quant_t(const void* x, int64_t n, float eps, float* partial, char* ct
   }
   if (vec && n <= kSmallElems) {
     const dim3 b(kFusedBlock);
-    const uint32_t spin = std::min(fused_spin_limit(), kColsSpinLimit);
+    const uint32_t spin = short_spin_limit(n * elem_bytes<DT>());
     if (n <= kSmallOneWg) {
       if (fp8) k_quant_tensor_small<DT, true, 4><<<dim3(1), b, 0, s>>>(x, n, eps, q, scale, ctl, spin);
       else k_quant_tensor_small<DT, false, 4><<<dim3(1), b, 0, s>>>(x, n, eps, q, scale, ctl, spin);
@@ -2497,7 +2521,7 @@ int cols_quant_t(const void* x, int64_t rows, int64_t cols, int64_t inner, float
                                s>>>(x, rows, static_cast<int>(cols / 8), sg.sl, sg.strips, sg.nrb,
                                     sg.RB, eps, q, scale, ctl,
                                     reinterpret_cast<unsigned long long*>(ctl + CBQ_WS_CTRL_BYTES),
-                                    std::min(fused_spin_limit(), kColsSpinLimit));
+                                    short_spin_limit(rows * cols * elem_bytes<DT>()));
       return launch_status(what);
     }
   }

@@ -60,8 +60,9 @@ enum { CBQ_OK = 0, CBQ_EINVAL = 1, CBQ_ELAUNCH = 2 };
  * status word stays 1 until cbq_tensor_quant_status_clear. Per-column quant
  * (cbq_quant_int8_channel, axis 1) and per-tensor quant of at most 2^19
  * elements use the block the same way, but a workgroup that gives up there
- * takes the maxima from x itself, after a few milliseconds: the results are
- * exact either way; the columns still set the status word. The other
+ * takes the missing maxima from x itself, after 40 us and as long again as x
+ * takes to be read: the results are exact either way; the columns still set the
+ * status word (a wait gave up: the call was slow, not wrong). The other
  * entry points leave the control block alone. The rest is per-call scratch. One
  * workspace serves one stream at a time: calls that overlap in time must not
  * share it. */

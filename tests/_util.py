@@ -79,3 +79,18 @@ def assert_array_equal(got, want, what: str = ""):
 def assert_scales_equal(got: np.ndarray, want: np.ndarray, what: str = ""):
     assert_array_equal(np.asarray(got, np.float32).view(np.uint32),
                        np.asarray(want, np.float32).view(np.uint32), what + " scale bits")
+
+
+def _suspect_view(dev: torch.device) -> torch.Tensor:
+    """The control block's word at byte 520 (the tag of the last call in which a
+    workgroup gave up waiting for the others, or 0) in the stream's workspace."""
+    from cublade_amd import _abi
+    return _abi._tensor_ws(dev)[520:524].view(torch.int32)
+
+
+def suspect_word(dev: torch.device) -> int:
+    return int(_suspect_view(dev).item())
+
+
+def set_suspect_word(dev: torch.device, value: int) -> None:
+    _suspect_view(dev).fill_(value)

@@ -21,7 +21,9 @@ import torch
 
 import oracle
 from cublade_amd import _abi
-from tests._util import assert_array_equal, assert_scales_equal, bits, from_bits
+from tests._util import (
+    assert_array_equal, assert_scales_equal, bits, from_bits, set_suspect_word, suspect_word,
+)
 
 pytestmark = pytest.mark.gpu
 
@@ -73,21 +75,27 @@ def test_cols_strip_special_values():
     check(xb, rows, cols, BF16)
 
 
-@pytest.mark.parametrize("rows,cols,code", [(1024, 2048, BF16), (700, 1000, F32)])
+@pytest.mark.parametrize("rows,cols,code", [(2048, 2048, BF16), (700, 1000, F32),
+                                            (11008, 512, F16), (20011, 72, BF16)])
 def test_cols_strip_gives_up_exact(rows, cols, code):
+    """The control block's suspect word tells that a workgroup gave up (shapes whose
+    strips have several row blocks; others need no exchange)."""
     xb = make(rows, cols, code, 17)
     xt = from_bits(xb.reshape(-1), code, "cuda").view(rows, cols)
     dev = xt.device
+    check(xb, rows, cols, code, xt)
     default = _abi.set_tensor_spin_limit(0)
     try:
         gave_up = 0
         for i in range(20):
+            set_suspect_word(dev, 0)
             check(xb, rows, cols, code, xt)
-            gave_up += _abi.tensor_quant_status(dev)
+            gave_up += suspect_word(dev) != 0
             _abi.clear_tensor_quant_status(dev)
     finally:
         _abi.set_tensor_spin_limit(default)
     print("calls in which a workgroup gave up:", gave_up, flush=True)
+    assert gave_up > 0
     for _ in range(3):
         check(xb, rows, cols, code, xt)
     assert _abi.tensor_quant_status(dev) == 0

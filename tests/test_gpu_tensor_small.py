@@ -17,7 +17,10 @@ from cublade_amd.bindings.hip.quantize_fp8 import quantize_per_tensor_fp8
 from cublade_amd.bindings.hip.quantize_int8 import (
     quantize_per_channel_int8, quantize_per_tensor_int8,
 )
-from tests._util import assert_array_equal, assert_fp8_equal, assert_scales_equal, bits, from_bits
+from tests._util import (
+    assert_array_equal, assert_fp8_equal, assert_scales_equal, bits, from_bits, set_suspect_word,
+    suspect_word,
+)
 
 pytestmark = pytest.mark.gpu
 F32, F16, BF16 = oracle.F32, oracle.F16, oracle.BF16
@@ -50,13 +53,20 @@ def test_tensor_small(n, code, fp8):
 
 def test_tensor_small_gives_up_exact():
     """With CUBLADE_CHECK_EXCHANGE=1 as well: an exact call never raises, also
-    after a column quant that set the status word."""
+    after a column quant that set the status word. The control block's suspect word
+    tells that a workgroup gave up."""
     dev = torch.device("cuda", torch.cuda.current_device())
     default = _abi.set_tensor_spin_limit(0)
     os.environ["CUBLADE_CHECK_EXCHANGE"] = "1"
     try:
-        for i in range(12):
+        check(65536, BF16, True, 3)
+        gave_up = 0
+        for i in range(24):
+            set_suspect_word(dev, 0)
             check([40960, 65536, 100003, (1 << 19) - 1][i % 4], BF16, i % 2 == 0, 5 + i, seed=i)
+            gave_up += suspect_word(dev) != 0
+        print("calls in which a workgroup gave up:", gave_up, flush=True)
+        assert gave_up > 0
         assert _abi.tensor_quant_status(dev) == 0
         quantize_per_channel_int8(torch.randn(4096, 512, device=dev), axis=1)
         check(65536, BF16, True, 3)
