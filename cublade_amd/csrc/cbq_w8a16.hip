@@ -86,6 +86,7 @@ struct GemmArgs {
   int full_tiles;           // split-K: tiles [0, full_tiles) run whole, the rest split
   const uint16_t* xp;       // k_decode: x as [M, ldx], 16-byte rows (x itself, or padded with zeros)
   int ldx;
+  int ldy;                  // row stride of y (N, or more for a part of the columns)
 };
 
 // Workgroup b of n goes to XCD b % 8; renumbered so that each XCD takes a
@@ -166,7 +167,7 @@ __device__ __forceinline__ void store_quad(const GemmArgs& a, const f4& acc, int
     for (int r = 0; r < 4; ++r)
       if (nb + r < a.N) v[r] += act_to_f32<ACT>(a.bias[nb + r]);
   }
-  uint16_t* dst = a.y + static_cast<int64_t>(m) * a.N + nb;
+  uint16_t* dst = a.y + static_cast<int64_t>(m) * a.ldy + nb;
   if (vec_store && nb + 3 < a.N) {
     *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_out<ACT>(v[0], v[1]),
                                                 pack2_out<ACT>(v[2], v[3]));
@@ -316,7 +317,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm(GemmArgs a) {
   }
 
   // Epilogue: lane owns y[m, nb .. nb+3] of each 16 x 16 tile.
-  const bool vec_store = (a.N % 4) == 0;
+  const bool vec_store = (a.ldy % 4) == 0;
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     const int m = m0 + wm * (BM / WGM) + j * 16 + (lane & 15);
@@ -794,7 +795,7 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
   }
   // Row-contiguous stores: 4 TN lanes cover one 32 TN-wide row (8 outputs
   // each).
-  const bool vec16 = (a.N % 8) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
+  const bool vec16 = (a.ldy % 8) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
   constexpr int LR = 4 * TN;
 #pragma unroll 4
   for (int u = 0; u < 2 * TM * TN; ++u) {
@@ -802,7 +803,7 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
     const int m = mw + row, n = nw + c8;
     if (m >= a.M || n >= a.N) continue;
     const u32x4 val = *reinterpret_cast<const u32x4*>(&ep[row * EPS + c8]);
-    uint16_t* dst = a.y + static_cast<int64_t>(m) * a.N + n;
+    uint16_t* dst = a.y + static_cast<int64_t>(m) * a.ldy + n;
     if (vec16 && n + 8 <= a.N) {
       *reinterpret_cast<u32x4*>(dst) = val;
     } else {
@@ -994,8 +995,8 @@ __global__ __launch_bounds__(kBlock) void k_splitk_reduce(GemmArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[u][r] += sbs[nr[u] + r];
     }
-    uint16_t* dst = a.y + static_cast<int64_t>(m) * a.N + nb;
-    if ((a.N % 4) == 0 && nb + 3 < a.N) {
+    uint16_t* dst = a.y + static_cast<int64_t>(m) * a.ldy + nb;
+    if ((a.ldy % 4) == 0 && nb + 3 < a.N) {
       *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_out<ACT>(v[u][0], v[u][1]),
                                                   pack2_out<ACT>(v[u][2], v[u][3]));
     } else {
@@ -1121,7 +1122,7 @@ __global__ __launch_bounds__(256) void k_skinny(GemmArgs a) {
 #pragma unroll
       for (int j = 0; j < TM; ++j) acc[i][j] += red[w][i][j][lane];
 
-  const bool vec_store = (a.N % 4) == 0;
+  const bool vec_store = (a.ldy % 4) == 0;
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     const int m = j * 16 + row;
@@ -1282,7 +1283,7 @@ __global__ __launch_bounds__(64 * kStreamWaves) void k_stream(GemmArgs a) {
   constexpr int RPR = kStreamLdsBytes / (kStreamWaves * TM * 1024) < RT
                           ? kStreamLdsBytes / (kStreamWaves * TM * 1024) : RT;
   f4* red = reinterpret_cast<f4*>(smem);
-  const bool vec_store = (a.N % 4) == 0;
+  const bool vec_store = (a.ldy % 4) == 0;
 #pragma unroll
   for (int r0 = 0; r0 < RT; r0 += RPR) {
     __syncthreads();
@@ -1306,7 +1307,7 @@ __global__ __launch_bounds__(64 * kStreamWaves) void k_stream(GemmArgs a) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) v[q] += act_to_f32<ACT>(braw[q]);
         }
-        uint16_t* dst = a.y + static_cast<int64_t>(m) * a.N + nq;
+        uint16_t* dst = a.y + static_cast<int64_t>(m) * a.ldy + nq;
         if (vec_store && nq + 3 < a.N) {
           *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_out<ACT>(v[0], v[1]),
                                                       pack2_out<ACT>(v[2], v[3]));
@@ -1437,8 +1438,8 @@ __global__ __launch_bounds__(1024) void k_stream1(GemmArgs a) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] += act_to_f32<ACT>(braw[q]);
     }
-    uint16_t* dst = a.y + static_cast<int64_t>(row) * a.N + nq;
-    if ((a.N % 4) == 0 && nq + 3 < a.N) {
+    uint16_t* dst = a.y + static_cast<int64_t>(row) * a.ldy + nq;
+    if ((a.ldy % 4) == 0 && nq + 3 < a.N) {
       *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_out<ACT>(v[0], v[1]),
                                                   pack2_out<ACT>(v[2], v[3]));
     } else {
@@ -1637,7 +1638,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < MT; ++j) red[((r * MT + j) * kDecWaves + wave) * 64 + lane] = acc[r][j];
   __syncthreads();
-  const bool vec_store = (a.N % 4) == 0;
+  const bool vec_store = (a.ldy % 4) == 0;
   for (int p = wave; p < RT * MT; p += kDecWaves) {
     const int r = p / MT, m = (p % MT) * 16 + row, nq = n0 + r * 16 + g * 4;
     if (m >= a.M || nq >= a.N) continue;
@@ -2187,11 +2188,24 @@ bool pad_direct(int64_t M, int64_t N, int64_t K) { return M <= 32 && N * K >= (8
 
 int64_t pad_align(int64_t v) { return cdiv(v, 256LL) * 256; }
 
+// The padded copies are made and used in parts where they would exceed these sizes:
+// rows of the weight (columns of y), and for each all rows of x in turn.
+constexpr int64_t kPadXBytes = int64_t(128) << 20, kPadWBytes = int64_t(256) << 20;
+
+// Rows per part, of rows of ld bytes: a multiple of 256, at least that many.
+int64_t pad_rows(int64_t rows, int64_t ld, int64_t cap) {
+  return std::min(rows, std::max<int64_t>(256, cap / ld / 256 * 256));
+}
+
 int64_t pad_bytes(int64_t M, int64_t N, int64_t K) {
   const int64_t kp = cdiv(K, 16LL) * 16;
-  const int64_t xb = pad_align(M * kp * 2);
-  if (pad_direct(M, N, K)) return xb;
-  return xb + pad_align(N * kp) + splitk_bytes(M, N, split_plan(M, N, kp));
+  if (pad_direct(M, N, K)) return pad_align(M * kp * 2);
+  const int64_t mr = pad_rows(M, kp * 2, kPadXBytes), nr = pad_rows(N, kp, kPadWBytes);
+  int64_t part = 0;   // of any part: whole ones and what is left of each side
+  for (const int64_t m : {mr, M % mr})
+    for (const int64_t n : {nr, N % nr})
+      if (m > 0 && n > 0) part = std::max(part, splitk_bytes(m, n, split_plan(m, n, kp)));
+  return pad_align(mr * kp * 2) + pad_align(nr * kp) + part;
 }
 
 // Whether the 32-bit sizes and offsets of the MFMA kernels hold.
@@ -2200,68 +2214,9 @@ bool pad_ok(int64_t M, int64_t N, int64_t K) {
          cdiv(M, 64) * cdiv(N, 64) < (1LL << 31) && (!pad_direct(M, N, K) || M * (K + 16) * 2 < (1LL << 31));
 }
 
-template <int ACT>
-int w8a16_t(const void* x, const int8_t* wq, const void* scales, const void* bias,
-            const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N, int64_t K,
-            void* ws, size_t ws_bytes, void* y, hipStream_t s);
-
-// bf16, M = 16, N = 9000, K = 5000 131.7 -> 24.7 us; M = 108, N = 7386, K = 4570
-// 333.8 -> 41.4; M = 2, N = 832, K = 5908 83.1 -> 15.6; M = 4096, N = 512, K = 1000
-// 191.7 -> 27.3; fp16 M = 16, N = K = 258 37.1 -> 6.4. Tiny products keep the one
-// launch of the general kernel (M = 1, N = 20, K = 10: 5.4 against 5.8 us).
-template <int ACT>
-int w8a16_padded(const void* x, const int8_t* wq, const void* scales, const void* bias,
-                 const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N,
-                 int64_t K, void* ws, size_t ws_bytes, void* y, hipStream_t s) {
-  const int64_t kp = cdiv(K, 16LL) * 16;
-  const bool direct = pad_direct(M, N, K);
-  uint8_t* const xd = static_cast<uint8_t*>(ws) + CBQ_WS_CTRL_BYTES;
-  uint8_t* const wd = xd + pad_align(M * kp * 2);
-  PadArgs p{};
-  p.src[0] = static_cast<const uint8_t*>(x);
-  p.dst[0] = xd;
-  p.rows[0] = M;
-  p.kb[0] = K * 2;
-  p.ld[0] = kp * 2;
-  p.src[1] = reinterpret_cast<const uint8_t*>(wq);
-  p.dst[1] = wd;
-  p.rows[1] = direct ? 0 : N;
-  p.kb[1] = K;
-  p.ld[1] = kp;
-  launch_pad(p, s);
-  if (!direct) {
-    // the control block's offset before the partials, which nothing here reads
-    const int64_t used = pad_align(M * kp * 2) + pad_align(N * kp);
-    return w8a16_t<ACT>(xd, reinterpret_cast<const int8_t*>(wd), scales, bias, oc, n_out, w_out, M,
-                        N, kp, static_cast<uint8_t*>(ws) + used, ws_bytes - used, y, s);
-  }
-  GemmArgs a{};
-  a.x = static_cast<const uint16_t*>(x);
-  a.xp = reinterpret_cast<const uint16_t*>(xd);
-  a.ldx = static_cast<int>(kp);
-  a.wq = wq;
-  a.scales = static_cast<const uint16_t*>(scales);
-  a.bias = static_cast<const uint16_t*>(bias);
-  a.oc = oc;
-  a.w_out = static_cast<const uint16_t*>(w_out);
-  a.y = static_cast<uint16_t*>(y);
-  a.M = static_cast<int>(M);
-  a.N = static_cast<int>(N);
-  a.K = static_cast<int>(K);
-  a.n_out = static_cast<int>(n_out);
-  launch_decode<ACT>(a, s);
-  return launch_status("cbq_w8a16_linear");
-}
-
-template <int ACT>
-int w8a16_t(const void* x, const int8_t* wq, const void* scales, const void* bias,
-            const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N, int64_t K,
-            void* ws, size_t ws_bytes, void* y, hipStream_t s) {
-  if (pad_ok(M, N, K) && aligned(x, 2) && aligned(y, 8) && ws &&
-      ws_bytes >= static_cast<size_t>(CBQ_WS_CTRL_BYTES + pad_bytes(M, N, K)))
-    return w8a16_padded<ACT>(x, wq, scales, bias, oc, n_out, w_out, M, N, K, ws, ws_bytes, y, s);
-  if (!mfma_path(M, N, K, x, wq, y))
-    return w8a16_general<ACT>(x, wq, scales, bias, oc, n_out, w_out, M, N, K, ws, ws_bytes, y, s);
+GemmArgs gemm_args(const void* x, const int8_t* wq, const void* scales, const void* bias,
+                   const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N,
+                   int64_t K, void* y, int64_t ldy) {
   GemmArgs a{};
   a.x = static_cast<const uint16_t*>(x);
   a.wq = wq;
@@ -2276,11 +2231,78 @@ int w8a16_t(const void* x, const int8_t* wq, const void* scales, const void* bia
   a.n_out = static_cast<int>(n_out);
   a.xp = a.x;
   a.ldx = a.K;
+  a.ldy = static_cast<int>(ldy);
+  return a;
+}
+
+// part: room for ws_bytes - CBQ_WS_CTRL_BYTES bytes of partial tiles, or null.
+template <int ACT>
+void w8a16_mfma(GemmArgs a, void* part, size_t ws_bytes, hipStream_t s) {
   DmaPlan plan{4, 0, 1};
-  const Kind kind = choose(M, N, K, n_out, ws ? ws_bytes : 0, plan);
-  if (kind == kTileDmaSplit)
-    a.part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + CBQ_WS_CTRL_BYTES);
+  const Kind kind = choose(a.M, a.N, a.K, a.n_out, part ? ws_bytes : 0, plan);
+  if (kind == kTileDmaSplit) a.part = static_cast<float*>(part);
   launch_kind<ACT>(kind, a, plan, s);
+}
+
+// bf16, M = 16, N = 9000, K = 5000 131.7 -> 24.7 us; M = 108, N = 7386, K = 4570
+// 333.8 -> 41.4; M = 2, N = 832, K = 5908 83.1 -> 15.6; M = 4096, N = 512, K = 1000
+// 191.7 -> 27.3; fp16 M = 16, N = K = 258 37.1 -> 6.4. Tiny products keep the one
+// launch of the general kernel (M = 1, N = 20, K = 10: 5.4 against 5.8 us).
+template <int ACT>
+int w8a16_padded(const void* x, const int8_t* wq, const void* scales, const void* bias,
+                 const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N,
+                 int64_t K, void* ws, size_t ws_bytes, void* y, hipStream_t s) {
+  const int64_t kp = cdiv(K, 16LL) * 16;
+  const bool direct = pad_direct(M, N, K);
+  const int64_t mr = pad_rows(M, kp * 2, kPadXBytes);
+  const int64_t nr = direct ? N : pad_rows(N, kp, kPadWBytes);
+  uint8_t* const xd = static_cast<uint8_t*>(ws) + CBQ_WS_CTRL_BYTES;
+  uint8_t* const wd = xd + pad_align(mr * kp * 2);
+  const int64_t used = pad_align(mr * kp * 2) + pad_align(nr * kp);
+  for (int64_t n0 = 0; n0 < N; n0 += nr)
+    for (int64_t m0 = 0; m0 < M; m0 += mr) {
+      const int64_t m = std::min(mr, M - m0), n = std::min(nr, N - n0);
+      PadArgs p{};
+      p.src[0] = static_cast<const uint8_t*>(x) + m0 * K * 2;
+      p.dst[0] = xd;
+      p.rows[0] = m;
+      p.kb[0] = K * 2;
+      p.ld[0] = kp * 2;
+      p.src[1] = reinterpret_cast<const uint8_t*>(wq) + n0 * K;
+      p.dst[1] = wd;
+      p.rows[1] = direct || m0 > 0 ? 0 : n;
+      p.kb[1] = K;
+      p.ld[1] = kp;
+      launch_pad(p, s);
+      uint16_t* const yp = static_cast<uint16_t*>(y) + m0 * N + n0;
+      if (direct) {
+        GemmArgs a = gemm_args(x, wq, scales, bias, oc, n_out, w_out, m, n, K, yp, N);
+        a.xp = reinterpret_cast<const uint16_t*>(xd);
+        a.ldx = static_cast<int>(kp);
+        launch_decode<ACT>(a, s);
+        continue;
+      }
+      const uint16_t* const b = static_cast<const uint16_t*>(bias);
+      const uint16_t* const wo = static_cast<const uint16_t*>(w_out);
+      w8a16_mfma<ACT>(gemm_args(xd, reinterpret_cast<const int8_t*>(wd),
+                                static_cast<const uint16_t*>(scales) + n0, b ? b + n0 : nullptr, oc,
+                                n_out, wo ? wo + n0 * n_out : nullptr, m, n, kp, yp, N),
+                      xd + used, ws_bytes - used, s);
+    }
+  return launch_status("cbq_w8a16_linear");
+}
+
+template <int ACT>
+int w8a16_t(const void* x, const int8_t* wq, const void* scales, const void* bias,
+            const int64_t* oc, int64_t n_out, const void* w_out, int64_t M, int64_t N, int64_t K,
+            void* ws, size_t ws_bytes, void* y, hipStream_t s) {
+  if (pad_ok(M, N, K) && aligned(x, 2) && aligned(y, 8) && ws &&
+      ws_bytes >= static_cast<size_t>(CBQ_WS_CTRL_BYTES + pad_bytes(M, N, K)))
+    return w8a16_padded<ACT>(x, wq, scales, bias, oc, n_out, w_out, M, N, K, ws, ws_bytes, y, s);
+  if (!mfma_path(M, N, K, x, wq, y))
+    return w8a16_general<ACT>(x, wq, scales, bias, oc, n_out, w_out, M, N, K, ws, ws_bytes, y, s);
+  w8a16_mfma<ACT>(gemm_args(x, wq, scales, bias, oc, n_out, w_out, M, N, K, y, N),
+                  ws ? static_cast<uint8_t*>(ws) + CBQ_WS_CTRL_BYTES : nullptr, ws_bytes, s);
   return launch_status("cbq_w8a16_linear");
 }
 

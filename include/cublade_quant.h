@@ -250,7 +250,9 @@ int cbq_dequant_int8_group_nd(const int8_t* q, const float* scale,
  * the control block, plus the split-K scratch of the kernel that dtype
  * selects. CBQ_F16 / CBQ_BF16 with K % 16 != 0: the rows of x, and unless M <=
  * 32 with a weight of 8 MB or more those of the weight, padded to a multiple of
- * 16, or the general kernel's partial sums if those are larger. CBQ_F16 /
+ * 16 (in parts of at most 128 MiB of x and 256 MiB of weight, one after another,
+ * reusing the workspace) and the split-K scratch of the padded product, or the
+ * general kernel's partial sums if those are larger. CBQ_F16 /
  * CBQ_BF16 (MFMA): for M > 64 when the
  * last wave of output tiles is short, the fp32 partial tiles of that wave
  * (ranges x tail tiles x 256 / 192 / 128 KiB for tiles of 256 / 192 / 128 x

@@ -54,3 +54,39 @@ def test_ragged_rows(M, K, N, n_out, dt):
                                   _abi.stream_handle(x.device)), "w8a16")
     err = (yg.double() - ref).abs()
     assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("M,K,N,n_out", [(70001, 1002, 67, 2), (40, 1002, 300001, 3)])
+def test_ragged_rows_in_parts(M, K, N, n_out):
+    """Padded copies past their caps are made in parts: rows of x (66560 and 3441 of
+    them), and rows of the weight (266240 and 33761, columns of y), with a workspace
+    of exactly the size asked for."""
+    from cublade_amd import _abi
+    dt, L, guard = torch.float16, _abi.lib(), 4096
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    print(f"[w8a16 ragged parts] M={M} K={K} N={N}", flush=True)
+    x = torch.randn(M, K, generator=g, device=DEV).to(dt)
+    w = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int16).to(torch.int8)
+    s = (torch.rand(N, generator=g, device=DEV) * 1e-3 + 1e-4).to(dt)
+    b = torch.randn(N, generator=g, device=DEV).to(dt)
+    oc = torch.tensor([0, K // 2, K - 1][:n_out], device=DEV)
+    w[:, oc] = 0
+    wo = (0.1 * torch.randn(N, n_out, generator=g, device=DEV)).to(dt)
+    need = L.cbq_w8a16_ws_bytes(M, N, K, n_out, _abi.F16)
+    assert need < 400 << 20
+    ws = torch.zeros(need + guard, dtype=torch.uint8, device=DEV)
+    ws[need:] = 0x5a
+    y = torch.empty(M, N, dtype=dt, device=DEV)
+    _abi.check(L.cbq_w8a16_linear(_abi.ptr(x), _abi.F16, _abi.ptr(w), _abi.ptr(s), _abi.ptr(b),
+                                  _abi.ptr(oc), n_out, _abi.ptr(wo), M, N, K, _abi.ptr(ws), need,
+                                  _abi.ptr(y), _abi.stream_handle(x.device)), "w8a16")
+    assert bool((ws[need:] == 0x5a).all())
+    for n0 in range(0, N, 60000):                    # float64 copies in parts
+        p = slice(n0, n0 + 60000)
+        wt, wot = w[p].double().t().contiguous(), wo[p].double().t().contiguous()
+        ref = (x.double() @ wt) * s[p].double() + b[p].double() + x[:, oc].double() @ wot
+        mag = (x.double().abs() @ wt.abs()) * s[p].double() + b[p].double().abs() \
+            + x[:, oc].double().abs() @ wot.abs()
+        bound = ref.abs() * 2.0 ** -11 * 1.01 + mag * (K + 8) * 2.0 ** -24 + 1e-6
+        err = (y[:, p].double() - ref).abs()
+        assert bool((err <= bound).all()), float((err / bound).max())

@@ -136,9 +136,13 @@ def test_workspace_sizes():
     assert L.cbq_w8a16_ws_bytes(500, 11008, 4096, 0, F32) == C + 500 * 4096 * 4 + 2048
     assert L.cbq_w8a16_ws_bytes(100000, 11008, 4096, 0, F32) == C + 12288 * (4096 * 4 + 4)
     assert L.cbq_w8a16_ws_bytes(1 << 20, 256, 64, 0, F32) <= C + (204 << 20)
-    # K % 16 != 0 takes the general kernel whatever the dtype
+    # K % 16 != 0: the general kernel's partial sums, fp16's padded rows of x are fewer
     assert L.cbq_w8a16_ws_bytes(16, 11008, 4090, 0, F16) == L.cbq_w8a16_ws_bytes(
         16, 11008, 4090, 0, F32)
+    # padded copies of x and of the weight in parts of at most 128 and 256 MiB
+    for M, N, K in ((262144, 4096, 4090), (40, 500000, 8190), (1 << 20, 200000, 1001)):
+        assert L.cbq_w8a16_ws_bytes(M, N, K, 0, F16) <= C + (128 << 20) + (256 << 20) + (64 << 20)
+    assert L.cbq_w8a16_ws_bytes(4096, 4096, 4090, 0, F16) == C + 4096 * 4096 * 3
     # 258 tiles of 256 x 256: one full wave whole, the 2 left over split 16 ways
     assert L.cbq_w8a16_ws_bytes(1536, 11008, 4096, 0, F16) == C + 16 * 2 * 256 * 1024
 
