@@ -34,6 +34,12 @@ __device__ __forceinline__ void dma_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// Orders a wave's LDS accesses for the compiler, where lanes read what other lanes of
+// the same wave wrote (the hardware runs a wave's LDS operations in order).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+}
+
 // A wave-uniform pointer in SGPRs (the DMA's scalar base operand).
 template <typename T>
 __device__ __forceinline__ const T* uniform_ptr(const T* p) {

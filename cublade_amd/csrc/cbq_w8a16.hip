@@ -793,6 +793,7 @@ __global__ __launch_bounds__(kDmaThreads) void k_gemm_dma(GemmArgs a) {
       }
     }
   }
+  wave_lds_fence();   // the wave's tile is written before lanes read each other's part
   // Row-contiguous stores: 4 TN lanes cover one 32 TN-wide row (8 outputs
   // each).
   const bool vec16 = (a.ldy % 8) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
@@ -1459,7 +1460,7 @@ __global__ __launch_bounds__(1024) void k_stream1(GemmArgs a) {
 // slower), D RT units in flight per wave (96 KiB or more per CU). A unit goes
 // through a 2 KiB stage of the wave's own in LDS into the MFMA layout (16-byte
 // chunk c of row r at c ^ (r & 7): no bank conflicts; LDS operations of a wave
-// are in order, so no barrier) and is widened and multiplied. x is staged by
+// are in order: compiler fences, no barrier) and is widened and multiplied. x is staged by
 // LDS DMA in chunks of KC = 1024 NBC columns (NBC blocks per wave; 16-byte chunk
 // c of row m at c ^ (m & 7)), double buffered: one barrier per chunk, then the
 // next chunk's DMA, waited for by count, so that the weight loads stay in
@@ -1616,11 +1617,13 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_decode(GemmArgs a) {
         }
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
+          wave_lds_fence();   // the last unit's fragments are read before the stage is written
           *reinterpret_cast<u32x4*>(st + wpos) = w[d][r][0];
           *reinterpret_cast<u32x4*>(st + 1024 + wpos) = w[d][r][1];
           if constexpr (ANY) {
             if (b == nblk - 1) place_last(r, w[d][r], st, wpos);
           }
+          wave_lds_fence();   // written by all lanes before it is read
           fw[0] = *reinterpret_cast<const u32x4*>(st + row * 128 + ((g ^ (row & 7)) << 4));
           fw[1] = *reinterpret_cast<const u32x4*>(st + row * 128 + (((g + 4) ^ (row & 7)) << 4));
           load(i + D, d, r);
