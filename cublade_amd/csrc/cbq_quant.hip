@@ -869,28 +869,27 @@ __global__ __launch_bounds__(kFusedBlock) void k_quant_cols_strip(
     float unused;
     const int ok = slot_wait<true>(ctl, tag, spin_limit, unused);
     if (t == 0 && ok) advance_gen(ctl, tag, b);
-    // Which row blocks to take from part: all, or after giving up those whose slot
-    // is there by now (decided once for the workgroup); the others' rows from x.
-    if (!ok) {
+    ColMax<DT> all;
+    if (ok) {
+      for (int p = tr; p < nrb; p += rps)
+        all.add(ld8_max<DT>(sp + static_cast<int64_t>(p) * NP * SW, SW, cc));
+    } else {
+      // gave up waiting: the row blocks whose slot is there by now (decided once for
+      // the workgroup) from part, the others' rows from x
       auto* slots = reinterpret_cast<unsigned long long*>(ctl + kCtlSlots);
       for (int p = t; p < nrb; p += kFusedBlock)
         s_there[p] = static_cast<uint32_t>(__hip_atomic_load(slots + p * strips + strip, __ATOMIC_RELAXED,
                                                              __HIP_MEMORY_SCOPE_AGENT) >> 32) == tag;
       __syncthreads();
-    }
-    ColMax<DT> all;
-    for (int p = tr; p < nrb; p += rps)
-      if (ok || s_there[p]) all.add(ld8_max<DT>(sp + static_cast<int64_t>(p) * NP * SW, SW, cc));
-    if (!ok && col_ok) {
       const int64_t c0 = (static_cast<int64_t>(strip) * SW + cc) * 8;
-      for (int p = 0; p < nrb; ++p)
-        if (!s_there[p])
-          for (int64_t rr = p * RB + tr, re = min((p + 1) * RB, rows); rr < re; rr += 2 * rps) {
-            const Raw8<DT> v0 = ld8<DT>(x, rr * c8 * 8 + c0);   // two: more would spill
-            const Raw8<DT> v1 = ld8<DT>(x, min(rr + rps, re - 1) * c8 * 8 + c0);
-            all.add(v0);
-            all.add(v1);
-          }
+      for (int p = 0; p < nrb; ++p) {
+        if (s_there[p]) {
+          if (p % rps == tr) all.add(ld8_max<DT>(sp + static_cast<int64_t>(p) * NP * SW, SW, cc));
+        } else if (col_ok) {
+          const int64_t re = min((p + 1) * RB, rows);
+          for (int64_t rr = p * RB + tr; rr < re; rr += rps) all.add(ld8<DT>(x, rr * c8 * 8 + c0));
+        }
+      }
     }
     all.across(SW);
     if (t % kWave < SW) {
@@ -2036,7 +2035,7 @@ uint32_t fused_spin_limit() { return spin_limit_var().load(std::memory_order_rel
 // each) for x of so many bytes. A workgroup with little to read waits for about the
 // time that x takes to be read (0.2 us per MiB, a third of a poll). With these limits
 // none of 100 uncontended calls gave up at any of 15 shapes up to 480 MiB; bf16
-// [11008, 4096] beside a kernel that holds 32 CUs for 8 ms takes 144 us (with 4096
+// [11008, 4096] beside a kernel that holds 32 CUs for 8 ms takes 159 us (with 4096
 // polls and the whole strip again 2300-2600; alone 29, as three launches 48).
 uint32_t short_spin_limit(int64_t bytes) {
   return std::min(fused_spin_limit(), 64u + static_cast<uint32_t>(bytes >> 21));
