@@ -57,11 +57,14 @@ def check_out_dtype(dtype: torch.dtype) -> int:
 
 def watch_exchange(dev: torch.device) -> bool:
     """Whether CUBLADE_CHECK_EXCHANGE=1 is in the environment; if so, clears
-    the status word of the stream's workspace (in stream order), so that
-    check_exchange after the call tells of that call alone."""
+    the status word of the stream's workspace where an earlier call left it set,
+    so that check_exchange after the call tells of that call alone. The word is
+    read first (which synchronises): a launch in front of every watched call
+    would change how its workgroups start."""
     if os.environ.get("CUBLADE_CHECK_EXCHANGE", "") in ("", "0"):
         return False
-    _abi.clear_tensor_quant_status(dev)
+    if _abi.tensor_quant_status(dev):
+        _abi.clear_tensor_quant_status(dev)
     return True
 
 
