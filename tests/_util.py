@@ -94,3 +94,39 @@ def suspect_word(dev: torch.device) -> int:
 
 def set_suspect_word(dev: torch.device, value: int) -> None:
     _suspect_view(dev).fill_(value)
+
+
+def w8a16_case(M, K, N, n_out, dt, seed, last_outlier=False):
+    """Random operands (x, w, s, b, oc, wo) of a W8A16 linear on the GPU, its float64
+    result, and a bound on the error per output: one rounding of the output to its
+    type plus K fp32 additions. The float64 copies of the weight are made in parts."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(M, K, generator=g, device="cuda").to(dt)
+    w = torch.randint(-127, 128, (N, K), generator=g, device="cuda", dtype=torch.int16).to(torch.int8)
+    s = (torch.rand(N, generator=g, device="cuda") * 1e-3 + 1e-4).to(dt)
+    b = torch.randn(N, generator=g, device="cuda").to(dt)
+    oc = wo = None
+    if n_out:
+        oc = torch.randperm(K, generator=g, device="cuda")[:n_out].sort().values
+        if last_outlier:
+            oc[-1] = K - 1
+        w[:, oc] = 0
+        wo = (0.1 * torch.randn(N, n_out, generator=g, device="cuda")).to(dt)
+    ref = torch.empty(M, N, dtype=torch.float64, device="cuda")
+    mag = torch.empty_like(ref)
+    for n0 in range(0, N, 65536):
+        p = slice(n0, n0 + 65536)
+        wt = w[p].double().t().contiguous()
+        ref[:, p] = (x.double() @ wt) * s[p].double() + b[p].double()
+        mag[:, p] = (x.double().abs() @ wt.abs()) * s[p].double() + b[p].double().abs()
+        if n_out:
+            wot = wo[p].double().t().contiguous()
+            ref[:, p] += x[:, oc].double() @ wot
+            mag[:, p] += x[:, oc].double().abs() @ wot.abs()
+    ulp = 2.0 ** (-11 if dt == torch.float16 else -8)
+    return (x, w, s, b, oc, wo), ref, ref.abs() * ulp * 1.01 + mag * (K + 8) * 2.0 ** -24 + 1e-6
+
+
+def assert_within(y, ref, bound):
+    err = (y.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())

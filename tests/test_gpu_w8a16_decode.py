@@ -9,8 +9,9 @@ from __future__ import annotations
 import pytest
 import torch
 
+from tests._util import assert_within, w8a16_case
+
 pytestmark = pytest.mark.gpu
-DEV = "cuda"
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
@@ -26,31 +27,8 @@ DEV = "cuda"
 def test_decode(M, K, N, n_out, dt):
     from cublade_amd.bindings.hip.w8a16 import w8a16_linear
     assert N * K >= 8 << 20
-    g = torch.Generator(device=DEV).manual_seed(M + K + N)
     print(f"[w8a16 decode] M={M} K={K} N={N} n_out={n_out} {dt}", flush=True)
-    x = torch.randn(M, K, generator=g, device=DEV).to(dt)
-    w = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int16).to(torch.int8)
-    s = (torch.rand(N, generator=g, device=DEV) * 1e-3 + 1e-4).to(dt)
-    b = torch.randn(N, generator=g, device=DEV).to(dt)
-    oc = wo = None
-    if n_out:
-        oc = torch.randperm(K, generator=g, device=DEV)[:n_out].sort().values
-        w[:, oc] = 0
-        wo = (0.1 * torch.randn(N, n_out, generator=g, device=DEV)).to(dt)
-    ref = torch.empty(M, N, dtype=torch.float64, device=DEV)
-    mag = torch.empty_like(ref)
-    for n0 in range(0, N, 65536):                     # float64 copies of the weight in parts
-        wt = w[n0:n0 + 65536].double().t().contiguous()
-        ref[:, n0:n0 + 65536] = x.double() @ wt
-        mag[:, n0:n0 + 65536] = x.double().abs() @ wt.abs()
-    ref = ref * s.double() + b.double()
-    mag = mag * s.double() + b.double().abs()
-    if n_out:
-        ref = ref + x[:, oc].double() @ wo.double().t().contiguous()
-        mag = mag + x[:, oc].double().abs() @ wo.double().abs().t().contiguous()
+    (x, w, s, b, oc, wo), ref, bound = w8a16_case(M, K, N, n_out, dt, M + K + N)
     y = w8a16_linear(x, w, s, b, oc, wo)
-    ulp = 2.0 ** (-11 if dt == torch.float16 else -8)
-    bound = ref.abs() * ulp * 1.01 + mag * (K + 8) * 2.0 ** -24 + 1e-6
-    err = (y.double() - ref).abs()
-    assert bool((err <= bound).all()), float((err / bound).max())
+    assert_within(y, ref, bound)
     assert torch.equal(w8a16_linear(x, w, s, b, oc, wo), y)

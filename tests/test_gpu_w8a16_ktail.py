@@ -8,6 +8,8 @@ from __future__ import annotations
 import pytest
 import torch
 
+from tests._util import assert_within, w8a16_case
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
@@ -20,27 +22,10 @@ DEV = "cuda"
     (3415, 560, 1673, 0), (40, 8240, 1024, 0)])
 def test_short_last_step(M, K, N, n_out, dt):
     from cublade_amd.bindings.hip.w8a16 import w8a16_linear
-    g = torch.Generator(device=DEV).manual_seed(M + K + N)
     print(f"[w8a16 k tail] M={M} K={K} N={N} n_out={n_out} {dt}", flush=True)
-    x = torch.randn(M, K, generator=g, device=DEV).to(dt)
-    w = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int16).to(torch.int8)
-    s = (torch.rand(N, generator=g, device=DEV) * 1e-3 + 1e-4).to(dt)
-    b = torch.randn(N, generator=g, device=DEV).to(dt)
-    oc = wo = None
-    ref = (x.double() @ w.double().t().contiguous()) * s.double() + b.double()
-    mag = (x.double().abs() @ w.double().abs().t().contiguous()) * s.double() + b.double().abs()
-    if n_out:
-        oc = torch.randperm(K, generator=g, device=DEV)[:n_out].sort().values
-        w[:, oc] = 0
-        wo = (0.1 * torch.randn(N, n_out, generator=g, device=DEV)).to(dt)
-        ref = (x.double() @ w.double().t().contiguous()) * s.double() + b.double() \
-            + x[:, oc].double() @ wo.double().t().contiguous()
-        mag = mag + x[:, oc].double().abs() @ wo.double().abs().t().contiguous()
+    (x, w, s, b, oc, wo), ref, bound = w8a16_case(M, K, N, n_out, dt, M + K + N)
     y = w8a16_linear(x, w, s, b, oc, wo)
-    ulp = 2.0 ** (-11 if dt == torch.float16 else -8)
-    bound = ref.abs() * ulp * 1.01 + mag * (K + 8) * 2.0 ** -24 + 1e-6
-    err = (y.double() - ref).abs()
-    assert bool((err <= bound).all()), float((err / bound).max())
+    assert_within(y, ref, bound)
     # rows past the end of x must not matter: the same rows inside a larger batch
     xl = torch.cat([x, torch.full((3, K), float("inf"), dtype=dt, device=DEV)])
     assert torch.equal(w8a16_linear(xl[:M].contiguous(), w, s, b, oc, wo), y)

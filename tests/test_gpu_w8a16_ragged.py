@@ -9,6 +9,8 @@ from __future__ import annotations
 import pytest
 import torch
 
+from tests._util import assert_within, w8a16_case
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
@@ -22,28 +24,10 @@ DEV = "cuda"
 def test_ragged_rows(M, K, N, n_out, dt):
     from cublade_amd import _abi
     from cublade_amd.bindings.hip.w8a16 import w8a16_linear
-    g = torch.Generator(device=DEV).manual_seed(M + K + N)
     print(f"[w8a16 ragged] M={M} K={K} N={N} n_out={n_out} {dt}", flush=True)
-    x = torch.randn(M, K, generator=g, device=DEV).to(dt)
-    w = torch.randint(-127, 128, (N, K), generator=g, device=DEV, dtype=torch.int16).to(torch.int8)
-    s = (torch.rand(N, generator=g, device=DEV) * 1e-3 + 1e-4).to(dt)
-    b = torch.randn(N, generator=g, device=DEV).to(dt)
-    oc = wo = None
-    if n_out:
-        oc = torch.randperm(K, generator=g, device=DEV)[:n_out].sort().values
-        oc[-1] = K - 1
-        w[:, oc] = 0
-        wo = (0.1 * torch.randn(N, n_out, generator=g, device=DEV)).to(dt)
-    ref = (x.double() @ w.double().t().contiguous()) * s.double() + b.double()
-    mag = (x.double().abs() @ w.double().abs().t().contiguous()) * s.double() + b.double().abs()
-    if n_out:
-        ref = ref + x[:, oc].double() @ wo.double().t().contiguous()
-        mag = mag + x[:, oc].double().abs() @ wo.double().abs().t().contiguous()
-    ulp = 2.0 ** (-11 if dt == torch.float16 else -8)
-    bound = ref.abs() * ulp * 1.01 + mag * (K + 8) * 2.0 ** -24 + 1e-6
+    (x, w, s, b, oc, wo), ref, bound = w8a16_case(M, K, N, n_out, dt, M + K + N, last_outlier=True)
     y = w8a16_linear(x, w, s, b, oc, wo)
-    err = (y.double() - ref).abs()
-    assert bool((err <= bound).all()), float((err / bound).max())
+    assert_within(y, ref, bound)
     # a workspace without room for the padded rows
     L = _abi.lib()
     ws = torch.zeros(_abi.WS_CTRL_BYTES, dtype=torch.uint8, device=DEV)
@@ -52,8 +36,7 @@ def test_ragged_rows(M, K, N, n_out, dt):
                                   _abi.ptr(b), _abi.ptr(oc), n_out, _abi.ptr(wo), M, N, K,
                                   _abi.ptr(ws), ws.numel(), _abi.ptr(yg),
                                   _abi.stream_handle(x.device)), "w8a16")
-    err = (yg.double() - ref).abs()
-    assert bool((err <= bound).all()), float((err / bound).max())
+    assert_within(yg, ref, bound)
 
 
 @pytest.mark.parametrize("M,K,N,n_out", [(70001, 1002, 67, 2), (40, 1002, 300001, 3)])
