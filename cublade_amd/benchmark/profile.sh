@@ -18,8 +18,8 @@
 #    of configs 1-5 (every suite kernel's HBM bytes per dispatch)
 # 4. the GPU clock under load (GRBM_GUI_ACTIVE over each dispatch's duration)
 #    and rocprof's derived MfmaUtil counter (MFMA busy cycles over active
-#    cycles x SIMDs) for the MFMA kernels: W8A16 (config 5) and the dense
-#    GEMM (f4)
+#    cycles x SIMDs) for the MFMA kernels: W8A16 (config 5, fp16 and fp32
+#    activations) and the dense GEMM (f4)
 # 5. bare stream ceilings (cublade_amd/benchmark/stream_ceiling.hip) and the
 #    MFMA-only matrix-core rate (cublade_amd/benchmark/mfma_ceiling.hip)
 # Summaries: OUTDIR/bench_c2_kernels.txt, OUTDIR/quant_int8_c2_traffic.json,
@@ -80,9 +80,9 @@ if want suite; then
   step "counter GRBM_GUI_ACTIVE: suite configs c2,c5,c5m,f4 (clock under load)"
   timeout -s KILL 300 rocprofv3 --pmc GRBM_GUI_ACTIVE --kernel-trace -d "$RAW/clk" -o suite -- \
     $PY -m cublade_amd.benchmark.suite --configs c2,c5,c5m,f4 --reps 3 --warmup 1 > "$LOGS/clk.log" 2>&1 || exit $?
-  step "counter MfmaUtil: suite configs c5,c5m,f4"
+  step "counter MfmaUtil: suite configs c5,c5m,c5f32,f4"
   timeout -s KILL 300 rocprofv3 --pmc MfmaUtil --kernel-trace -d "$RAW/mfma" -o suite -- \
-    $PY -m cublade_amd.benchmark.suite --configs c5,c5m,f4 --reps 3 --warmup 1 > "$LOGS/mfma.log" 2>&1 || exit $?
+    $PY -m cublade_amd.benchmark.suite --configs c5,c5m,c5f32,f4 --reps 3 --warmup 1 > "$LOGS/mfma.log" 2>&1 || exit $?
 
 fi
 if want ceil; then
@@ -142,19 +142,20 @@ if want suite; then
     echo "# rocprof derived counter MfmaUtil = sum(SQ_VALU_MFMA_BUSY_CYCLES) / (max(GRBM_GUI_ACTIVE) * SIMDs) * 100,"
     echo "# per kernel: mean and median over dispatches, then the values in dispatch order (the first is the"
     echo "# suite's warm-up call): W8A16 (suite configs c5 and c5m, M = 16 / 256 / 768 / 1536 / 4096 and"
-    echo "# 1024 / 2048 / 3072) and the dense GEMM (f4, 8192^3)"
-    echo "# command: rocprofv3 --pmc MfmaUtil --kernel-trace -d RAW/mfma -o suite -- python -u -m cublade_amd.benchmark.suite --configs c5,c5m,f4 --reps 3 --warmup 1"
-    $R counters "$RAW/mfma/suite_results.db" | grep -E "k_gemm_dma|k_stream|k_skinny|k_gemm<|k_mm_dma|Cijk"
+    echo "# 1024 / 2048 / 3072; c5f32, M = 16 / 256 / 4096) and the dense GEMM (f4, 8192^3)"
+    echo "# command: rocprofv3 --pmc MfmaUtil --kernel-trace -d RAW/mfma -o suite -- python -u -m cublade_amd.benchmark.suite --configs c5,c5m,c5f32,f4 --reps 3 --warmup 1"
+    $R counters "$RAW/mfma/suite_results.db" | grep -E "k_gemm_dma|k_gemm_f32|k_decode|k_stream|k_skinny|k_gemm<|k_mm_dma|Cijk"
     echo
     echo "# dispatches by W8A16 shape (N = 11008, K = 4096, config-5 operands; order: c5 then c5m):"
-    echo "#   M = 16    k_stream1<1, 3>                          (weight streaming, HBM-bound)"
-    echo "#   M = 256   k_gemm_dma<1, false, 2, false, 1, 2>     (172 tiles of 128 x 128, one round, no split)"
-    echo "#   M = 768   k_gemm_dma<1, false, 3, false, 2, 2>     first 4 values (172 tiles of 192 rows, one wave)"
-    echo "#   M = 1536  k_gemm_dma<1, true, 4, false, 2, 2>      first 4 values (256 tiles whole + 2 over 16 ranges)"
-    echo "#   M = 4096  k_gemm_dma<1, false, 4, false, 2, 2>     first 4 values (688 tiles, 2.69 waves)"
-    echo "#   M = 1024  k_gemm_dma<1, false, 4, false, 2, 2>     last 4 values (172 tiles of 256 rows, one wave)"
-    echo "#   M = 2048  k_gemm_dma<1, false, 3, false, 2, 2>     last 4 values (473 tiles of 192 rows)"
-    echo "#   M = 3072  k_gemm_dma<1, true, 4, false, 2, 2>      last 4 values (512 tiles whole + the tail split)"
+    echo "#   M = 16    k_stream1<1>                                    (weight streaming, HBM-bound)"
+    echo "#   M = 256   k_gemm_dma<1, false, 2, 1, 2, false>            (172 tiles of 128 x 128, one round, no split)"
+    echo "#   M = 768   k_gemm_dma<1, false, 3, 2, 2, false>            first 4 values (172 tiles of 192 rows, one wave)"
+    echo "#   M = 1536  k_gemm_dma<1, true, 4, 2, 2, false>             first 4 values (256 tiles whole + 2 over 16 ranges)"
+    echo "#   M = 4096  k_gemm_dma<1, false, 4, 2, 2, false>            first 4 values (688 tiles, 2.69 waves)"
+    echo "#   M = 1024  k_gemm_dma<1, false, 4, 2, 2, false>            last 4 values (172 tiles of 256 rows, one wave)"
+    echo "#   M = 2048  k_gemm_dma<1, false, 3, 2, 2, false>            last 4 values (473 tiles of 192 rows)"
+    echo "#   M = 3072  k_gemm_dma<1, true, 4, 2, 2, false>             last 4 values (512 tiles whole + the tail split)"
+    echo "#   fp32 x  k_gemm_f32: M = 16 <2, 2, true>, M = 256 <2, 4, false>, M = 4096 <3, 4, false>"
     echo "# dense GEMM (f4): k_mm_dma<0, 0, ...> int8 (B [N, K] read in place, then [K, N]), k_mm_dma<1, 1, ...>"
     echo "# fp16 -> fp32; Cijk_* are hipBLASLt's kernels for torch._int_mm and torch.matmul on the same shapes"
   } > "$OUT/mfma_util.txt" || exit $?
