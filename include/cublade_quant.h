@@ -259,7 +259,7 @@ int cbq_dequant_int8_group_nd(const int8_t* q, const float* scale,
  * 256; at most 16 ranges and at most one partial tile per CU, i.e. <= 64 MiB
  * on MI355X; the same with outlier columns), else nothing. CBQ_F32 on the
  * matrix-core path (see cbq_w8a16_linear): two 16-bit planes of x (4 M K
- * bytes), 4 bytes per row and, when K is split, 4 bytes per output and
+ * bytes), 12 bytes per row and, when K is split, 4 bytes per output and
  * k-range (at most 16 and at most one tile per CU). A larger M runs in chunks
  * of rows (multiples of 256, one after another, reusing the workspace) whose
  * planes stay within 192 MiB (or of 256 rows where those alone exceed it). Other CBQ_F32
@@ -282,8 +282,8 @@ size_t cbq_w8a16_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t n_out, int ac
  * hardware) with K % 64 == 0, no outlier columns, M > 64 or a weight of at
  * least 8 MB, and a workspace of cbq_w8a16_ws_bytes also runs on MFMA: x as two
  * fp16 planes under a power-of-two scale per row, 16 to 22 significant bits of
- * every element (rows whose non-zero magnitudes span more than 2^34 as three
- * bf16 numbers instead, exact, at up to 2.5 times the time), fp32
+ * every element (those outside a band of 2^35 that holds most of their row as
+ * three bf16 numbers, exact, which costs time only where there are any), fp32
  * accumulation; other CBQ_F32 calls,
  * unaligned operands and fp16 / bf16 with K % 16 != 0 and no room in ws for the
  * padded rows run a tiled fp32-FMA kernel. K == 0

@@ -5,8 +5,8 @@ Shapes reach each tile (64 rows x 128 / 256 / 384 columns, 128 x 64 / 128 / 192)
 whole and split over K, with partial tiles in M and N, rows that a workgroup does
 not hold in registers (K > 16384), and calls of several row chunks. The bound per
 output: an element of these rows keeps 21 significant bits or more (two fp16 planes
-down to 2^-29 of the row's largest, three bf16 ones in rows that span more than
-2^34), and the fp32 sums add a few 2^-24 of sum |x w s|; 2^-20 of that sum in all.
+down to 2^-29 of the row's largest, three bf16 ones for elements outside the row's
+band), and the fp32 sums add a few 2^-24 of sum |x w s|; 2^-20 of that sum in all.
 """
 from __future__ import annotations
 
@@ -85,8 +85,8 @@ def test_f32_spikes_and_special_rows():
 @pytest.mark.parametrize("M", [1080, 1500, 2110])
 def test_f32_row_chunks(M):
     """K = 40000: 1024 rows per chunk. One chunk with the remainder merged, two, and
-    two of which the second is longer; a wide and a narrow row in the second; a
-    workspace of exactly the size asked for."""
+    two of which the second is longer; a row with elements outside its band and one
+    without in the second; a workspace of exactly the size asked for."""
     from cublade_amd import _abi
     K, N, guard = 40000, 64, 4096
     L = _abi.lib()

@@ -103,7 +103,7 @@ def test_workspace_sizes():
     assert big >= C + 8192 * 4 * 2 and big < 64 << 20
     F16, F32 = _abi.F16, _abi.F32
     # M <= 16, fp16: the weight-streaming kernel, no partials. fp32 activations:
-    # the larger of the matrix-core path's needs (two 16-bit planes of x, 4 bytes
+    # the larger of the matrix-core path's needs (two 16-bit planes of x, 12 bytes
     # per row, fp32 sums of the k-ranges) and the general kernel's (16 k-ranges of
     # [16, 11008] fp32 partial sums)
     assert L.cbq_w8a16_ws_bytes(16, 11008, 4096, 0, F16) == C
@@ -129,12 +129,12 @@ def test_workspace_sizes():
     assert L.cbq_w8a16_ws_bytes(64, 4096, 11008, 0, F16) == C + 11 * 16 * 128 * 1024
     assert L.cbq_w8a16_ws_bytes(32, 4096, 11008, 0, F16) == C + 11 * 16 * 128 * 1024
     # M = 24: k_stream<2>, no MFMA partials; fp32: the general kernel's 16 ranges of
-    # [24, 4096] fp32 again; M = 500: whole tiles, the planes and row exponents alone;
+    # [24, 4096] fp32 again; M = 500: whole tiles, the planes and the rows' exponents and masks;
     # rows past 192 MiB of planes in chunks (12288 rows at K = 4096)
     assert L.cbq_w8a16_ws_bytes(24, 4096, 11008, 0, F16) == C
     assert L.cbq_w8a16_ws_bytes(24, 4096, 11008, 0, F32) == C + 16 * 24 * 4096 * 4
-    assert L.cbq_w8a16_ws_bytes(500, 11008, 4096, 0, F32) == C + 500 * 4096 * 4 + 2048
-    assert L.cbq_w8a16_ws_bytes(100000, 11008, 4096, 0, F32) == C + 12288 * (4096 * 4 + 4)
+    assert L.cbq_w8a16_ws_bytes(500, 11008, 4096, 0, F32) == C + 500 * 4096 * 4 + 2048 + 4096
+    assert L.cbq_w8a16_ws_bytes(100000, 11008, 4096, 0, F32) == C + 12288 * (4096 * 4 + 12)
     assert L.cbq_w8a16_ws_bytes(1 << 20, 256, 64, 0, F32) <= C + (204 << 20)
     # K % 16 != 0: the general kernel's partial sums, fp16's padded rows of x are fewer
     assert L.cbq_w8a16_ws_bytes(16, 11008, 4090, 0, F16) == L.cbq_w8a16_ws_bytes(
